@@ -62,7 +62,9 @@ enum {
  *   x          [M, K] bf16, row stride ldx >= K, ldx % 8 == 0, 16-byte aligned
  *   w          [N, K] bf16, row stride ldw >= K, ldw % 8 == 0, 16-byte aligned
  *   y          [M, Nout] bf16, row stride ldy >= Nout; must not overlap x, w or workspace
- *   M >= 1 (rows beyond 64 are processed in chunks of 64), N >= 1, K >= 8, K % 8 == 0
+ *   M >= 1, N >= 1, K >= 8, K % 8 == 0.  More than 64 rows run in launches of
+ *              up to 128 rows while more than 64 are left (the tile kernel, one
+ *              pass over w each), then one of up to 64
  *   epilogue   KRK_EPILOGUE_NONE or KRK_EPILOGUE_SILU_MUL
  *   workspace  device memory of at least krk_gemm_workspace_bytes(M, N, K, epilogue)
  *              bytes (may be NULL when that is 0).  It must be zero-filled once
@@ -152,7 +154,10 @@ typedef struct krk_gemm_config {
  * krk_gemm_plan — the configuration krk_gemm_bf16 uses for this shape (the
  * static shape -> kernel table that stands in for the reference's warm-up
  * pickers, engine/kernels/gemm.py:417-458, 461-498).  Returns KRK_OK or a
- * negative error for an invalid shape.
+ * negative error for an invalid shape.  For more than 64 rows it describes the
+ * launches of up to 64 rows; calls with it (or with no configuration) take
+ * their larger launches on the tile kernel, whose own tiles follow from the
+ * shape.  Any other configuration runs in launches of up to 64 rows.
  */
 int krk_gemm_plan(int M, int N, int K, int epilogue, krk_gemm_config* out);
 

@@ -23,6 +23,7 @@
 #include "krk_select.h"
 #include "krk_slice.h"
 #include "krk_stream.h"
+#include "krk_tile.h"
 #include "krk_valu.h"
 
 namespace {
@@ -257,8 +258,8 @@ int stream_xs(int MT, int nst);
 // MFMA_LDS k per stage when the caller or the table does not choose one.
 inline int default_kc(int MT, int NT) { return krk::mfma_lds_kc_ok(MT, NT, 512) ? 512 : 256; }
 
-void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
-    const int Mc = M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch;
+// The plan of launches of up to 64 rows.
+void chunk_config(int Mc, int N, int K, int epilogue, krk_gemm_config* c) {
     const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
     const int mt = cdiv(Mc, 16);
     const int KST = cdiv(K, 512);
@@ -326,6 +327,22 @@ void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
         while (nblocks * r.splits < 192 && r.splits < 4 && KST >= 2 * (r.splits + 1)) ++r.splits;
     }
     *c = r;
+}
+
+// Splits of a plan for more than 64 rows: its workspace also holds the tile
+// kernel's partial sums, 128 rows x splits / 2 of them (tall_plan below).
+// Only plans that split K anyway take more splits, as many as the static
+// scratch of krk_gemm_bf16_noalloc holds; the block counters keep their place
+// (the block geometry does not change).
+constexpr int kTallPlanSplits = 6;
+
+void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
+    chunk_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue, c);
+    if (M <= kMaxRowsPerLaunch || c->kernel != KRK_KERNEL_MFMA_LDS || c->splits == 1) return;
+    const size_t one = (size_t)kMaxRowsPerLaunch * N * sizeof(float);
+    while (c->splits < kTallPlanSplits && c->splits < cdiv(K, 512) &&
+           (c->splits + 1) * one <= KRK_NOALLOC_SCRATCH_BYTES - KRK_NOALLOC_COUNTER_BYTES)
+        ++c->splits;
 }
 
 // MFMA_LDS keeps `unroll` stages of row pieces in registers; three stages fit
@@ -861,6 +878,87 @@ int dispatch_slice(const LaunchArgs& a, const krk_gemm_config& c, int nblocks, h
                             : dispatch_slice_kc<64>(a, v, c.unroll, nblocks, s);
 }
 
+// How one launch of the tile kernel cuts `rows` (65..128) rows: tiles, output
+// channels per block and K splits, whose partial sums fit part_bytes.
+struct TallPlan {
+    int mt, nt, cb, splits, nblk;
+};
+
+// The cheapest cut under a linear model of the measured times (MI355X, 96 and
+// 128 rows of the Qwen3-4B projections): a CU takes in 47 KB of x and W
+// together per us, a launch costs 3 us beside that, and a split K the second
+// launch's 4 us.  The model puts qkv, gate_up and lm_head on whole K (qkv
+// M = 128: 17.0 us against 18.4 with 2 splits) and o and down on the most
+// splits their workspace holds (o: 16.2 with 4 splits, 24 unsplit).  Blocks
+// are cut to one per CU where the tiles allow it.
+TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
+    const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
+    const int Nout = silu ? N / 2 : N;
+    const int unit = silu ? 8 : 16;  // output channels of a W tile
+    const int stages = cdiv(K, krk::kTileKC);
+    TallPlan best{};
+    double best_us = 0.0;
+    const int mt = rows > 96 ? 8 : 6;
+    for (int sp = 1; sp <= krk::kTileMaxSplits && sp <= stages; ++sp) {
+        // One block per CU and split, in the 4 channels of a store.
+        const int64_t one = (((int64_t)Nout * sp + kCuCount - 1) / kCuCount + 3) / 4 * 4;
+        for (int nt = 2; nt <= krk::kTileMaxNT; ++nt)
+            for (int cb : {(int)(one < nt * unit ? one : nt * unit), nt * unit}) {
+                if (nt > 2 && cb <= (nt - 1) * unit) continue;  // fewer tiles hold it
+                TallPlan p{mt, nt, cb, sp, cdiv(Nout, cb)};
+                if (sp > 1 && sp * krk::tile_part_bytes(mt, nt, p.nblk) > part_bytes) continue;
+                const double bytes = 16.0 * (mt + nt) * 2 * krk::kTileKC * cdiv(stages, sp);
+                const double us = 3.0 + cdiv(p.nblk * sp, kCuCount) * bytes / 47e3 + (sp > 1 ? 4.0 : 0.0);
+                if (!best.mt || us < best_us) {
+                    best = p;
+                    best_us = us;
+                }
+            }
+    }
+    return best;
+}
+
+template <int MT, int NT, bool SILU>
+int launch_tile(const krk::TileArgs& a, hipStream_t stream) {
+    constexpr int D = krk::tile_depth(MT, NT, kLdsMax);
+    constexpr size_t shm = krk::tile_lds_bytes(MT, NT, D);
+    const void* fn = reinterpret_cast<const void*>(&krk::tile_gemm_kernel<MT, NT, D, SILU>);
+    static std::atomic<uint64_t> done{0};
+    hipError_t e = ensure_lds_limit(fn, (int)shm, done);
+    if (e != hipSuccess) return hip_status(e, "tile_gemm_kernel LDS attribute");
+    void* args[] = {(void*)&a};
+    e = hipLaunchKernel(fn, dim3(a.nblk * a.splits), dim3(64 * krk::tile_waves(MT)), args, shm, stream);
+    if (e != hipSuccess || a.splits == 1) return hip_status(e, "tile_gemm_kernel launch");
+    int mt = MT, nt = NT;
+    void* rargs[] = {(void*)&a, (void*)&mt, (void*)&nt};
+    const void* rfn = a.splits == 2   ? reinterpret_cast<const void*>(&krk::tile_reduce_kernel<2, SILU>)
+                      : a.splits == 3 ? reinterpret_cast<const void*>(&krk::tile_reduce_kernel<3, SILU>)
+                                      : reinterpret_cast<const void*>(&krk::tile_reduce_kernel<4, SILU>);
+    e = hipLaunchKernel(rfn, dim3(cdiv(a.nblk * MT * NT * 64, krk::kTileReduceThreads)),
+                        dim3(krk::kTileReduceThreads), rargs, 0, stream);
+    return hip_status(e, "tile_reduce_kernel launch");
+}
+
+template <int MT, bool SILU>
+int dispatch_tile_n(const krk::TileArgs& a, int nt, hipStream_t s) {
+    switch (nt) {
+        case 2: return launch_tile<MT, 2, SILU>(a, s);
+        case 3: return launch_tile<MT, 3, SILU>(a, s);
+        case 4: return launch_tile<MT, 4, SILU>(a, s);
+        case 5: return launch_tile<MT, 5, SILU>(a, s);
+    }
+    return fail(KRK_ERR_UNSUPPORTED, "tile kernel with %d weight tiles", nt);
+}
+
+// y of a.M (65..128) rows; part: part_bytes of workspace for split sums.
+int dispatch_tile(const LaunchArgs& a, int epilogue, size_t part_bytes, hipStream_t s) {
+    const TallPlan p = tall_plan(a.M, a.N, a.K, epilogue, part_bytes);
+    const krk::TileArgs t{a.x, a.ldx, a.w, a.ldw, a.y, a.ldy, a.M, a.N, a.K, p.splits, p.cb, p.nblk, a.part};
+    if (epilogue == KRK_EPILOGUE_SILU_MUL)
+        return p.mt == 8 ? dispatch_tile_n<8, true>(t, p.nt, s) : dispatch_tile_n<6, true>(t, p.nt, s);
+    return p.mt == 8 ? dispatch_tile_n<8, false>(t, p.nt, s) : dispatch_tile_n<6, false>(t, p.nt, s);
+}
+
 template <int MX, int R, int D, bool SILU, bool NORM = false, bool SEL = false>
 int launch_valu(const LaunchArgs& a, int nblocks, int waves, hipStream_t stream, krk::NormArgs na = {},
                 krk::SelectArgs sa = {}) {
@@ -1185,7 +1283,20 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
         xin = nrows;
         ldin = ldn;
     }
-    for (int m0 = 0; m0 < M; m0 += kMaxRowsPerLaunch) {
+    // More than 64 rows under the plan (a configuration equal to it included):
+    // launches of up to 128 rows on the tile kernel while more than 64 are left.
+    bool tall = M > kMaxRowsPerLaunch && !fused;
+    if (tall) {
+        krk_gemm_config plan;
+        auto_config(M, N, K, epilogue, &plan);
+        plan.prologue = c.prologue;
+        tall = !memcmp(&plan, &c, sizeof c);
+    }
+    int rows = 0;
+    for (int m0 = 0; m0 < M; m0 += rows) {
+        const bool tile = tall && M - m0 > kMaxRowsPerLaunch;
+        const int most = tile ? krk::kTileMaxRows : kMaxRowsPerLaunch;
+        rows = M - m0 < most ? M - m0 : most;
         LaunchArgs a;
         a.x = xin + (int64_t)m0 * ldin;
         a.ldx = ldin;
@@ -1193,14 +1304,16 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
         a.ldw = ldw;
         a.y = static_cast<uint16_t*>(y) + (int64_t)m0 * ldy;
         a.ldy = ldy;
-        a.M = (M - m0) < kMaxRowsPerLaunch ? (M - m0) : kMaxRowsPerLaunch;
+        a.M = rows;
         a.N = N;
         a.K = K;
         a.splits = c.splits;
         a.part = part;
         a.ctr = ctr;
         a.cb = g.cb;
-        if (fused) {
+        if (tile) {
+            rc = dispatch_tile(a, epilogue, part ? (size_t)c.splits * kMaxRowsPerLaunch * N * sizeof(float) : 0, st);
+        } else if (fused) {
             // This chunk's rows of d and xout.
             krk::NormArgs nc = na;
             nc.d += (int64_t)m0 * na.ldd;
