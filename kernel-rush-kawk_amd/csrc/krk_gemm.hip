@@ -255,8 +255,230 @@ inline int valu_depth(int MX, int R, int blocks) {
 
 int stream_xs(int MT, int nst);
 
+// Dynamic LDS a gfx950 workgroup may use: 160 KB less room for the kernels'
+// static __shared__ variables.
+constexpr size_t kLdsMax = 163840 - kLdsReserve;
+
+// MFMA_LDS keeps `unroll` stages of row pieces in registers; three stages fit
+// 256 VGPRs without spilling up to this many 16-row tiles (m + n).
+constexpr int kLdsPf3MaxTiles = 6;
+constexpr bool mfma_lds_pf3(int MT, int NT) { return MT + NT <= kLdsPf3MaxTiles; }
 // MFMA_LDS k per stage when the caller or the table does not choose one.
 inline int default_kc(int MT, int NT) { return krk::mfma_lds_kc_ok(MT, NT, 512) ? 512 : 256; }
+
+// Plans of the shapes the table does not hold (other tensor-parallel degrees,
+// other models' projections).  From sweeps of every candidate on 23 shapes
+// (N 400-38000, K 1024-9728, plain and SwiGLU) at 1-64 rows on an MI355X,
+// graph replay over rotating weights; times below in us.  Against the rule
+// before it, which split K until 200-600 workgroups ran, 500 random shapes
+// (N 256-24576, K 512-10240, 1-64 rows) run 1.33x as fast (geometric mean),
+// none of them more than 3% slower.
+//
+// All rules cut the channels into one block per CU, or into whole rounds of
+// 256 blocks, and leave K whole: a split pays 3.4 us (2 splits) to 8 us (8)
+// for its fix-up, more than the CUs it fills give back except where there
+// are few channels and K is long.
+inline int round8(int v) { return (v + 7) / 8 * 8; }
+// Share of 256-block rounds that `blocks` fill.
+inline double round_fill(int blocks) { return (double)blocks / ((double)cdiv(blocks, kCuCount) * kCuCount); }
+// Channels per block (a multiple of 8, at most `most`) for whole rounds.
+inline int even_channels(int Nout, int most) {
+    const int rounds = cdiv(Nout, kCuCount * most);
+    return round8(cdiv(Nout, kCuCount * rounds));
+}
+
+// VALU: a block of `waves` waves, one or two W rows each.
+//   * One row per wave: plain, M = 1 past 2560 channels (18280 x 3000: 19.0
+//     against 20.9 with two) and below 2048; else two (3072 x 2560, M = 2:
+//     4.65 against 4.92).
+//   * Waves: as many as make one round of blocks, where eight can; with more
+//     rounds the count whose blocks fill them best (N = 2432 SwiGLU channels,
+//     M = 2: 6.44 with 5 waves, 6.87 with 4).  With x in LDS (M >= 3) the
+//     waves of a block share it: eight, plain (2560 x 2048, M = 4: 4.6
+//     against 4.8) unless a short K ends in part of a block (9518 x 2240, M =
+//     3: 10.2 with 4 waves of one row, 10.7 with 8 of two), and SwiGLU where x
+//     leaves a CU fewer than three blocks
+//     (12000 channels, K = 4096, M = 6: 33.5 with 8, 41.6 with 4).
+//   * K is split only where a few blocks would each walk a long K (307 SwiGLU
+//     channels, K = 9600, M = 6: 9.6 with 8 splits, 14.6 whole), and where x
+//     would leave a CU one or two blocks over 16 or more blocks of k.
+//   * Depth: blocks that fit one round hold all of a row in flight; with more
+//     rounds other workgroups cover the latency and a depth past 7 only costs
+//     occupancy (6810 x 7120, M = 1: 16.8 with 2 in flight, 23.2 with 19;
+//     12288 x 4096: 15.8 with 4, 17.0 with 8).
+void valu_rule(int Mc, int N, int K, bool silu, krk_gemm_config* r) {
+    const int Nout = silu ? N / 2 : N;
+    const int nb = cdiv(K, krk::kValuBlock);
+    r->kernel = KRK_KERNEL_VALU;
+    r->m_tiles = valu_mx(Mc);
+    r->n_tiles = silu || (N > 8 * kCuCount && (Mc > 1 || N <= 10 * kCuCount || (N <= 16 * kCuCount && nb > 8))) ? 2 : 1;
+    const int per_wave = silu ? 1 : r->n_tiles;
+    r->splits = 1;
+    const int quads = cdiv(Nout, 4 * per_wave);  // blocks of 4 waves
+    const bool starved = Mc >= 2 && quads < 192 && nb >= (Mc == 2 ? 10 : 8);
+    const size_t fit = Mc >= 3 && nb >= 16 ? kLdsBudget : kLdsMax;
+    while (r->splits < nb && r->splits < 32 &&
+           ((starved && quads * r->splits < 600) || krk::valu_lds_bytes(r->m_tiles, cdiv(nb, r->splits)) > fit))
+        ++r->splits;
+    const int per = cdiv(nb, r->splits);
+    if (r->splits > 1) {
+        r->waves = 4;
+        r->unroll = valu_depth(r->m_tiles, r->n_tiles, per);
+        return;
+    }
+    const size_t lds = krk::valu_lds_bytes(r->m_tiles, per);
+    const int one_round = cdiv(Nout, kCuCount * per_wave);  // waves of a single round's blocks
+    const bool single = one_round <= krk::kValuMaxWaves;
+    const bool whole = K % krk::kValuBlock == 0;
+    if (Mc >= 3 && !silu && !single && !whole && nb <= 5) {
+        r->n_tiles = Mc <= 4 ? 1 : 2;
+        r->waves = 4;
+    } else if (Mc >= 3 && (!silu || lds > kLdsMax / 3)) {
+        r->waves = krk::kValuMaxWaves;
+    } else if (single) {
+        r->waves = one_round < 4 ? 4 : one_round;
+    } else {
+        r->waves = 4;
+        if (Mc <= 4 && quads <= 8 * kCuCount && nb > 3)
+            for (int wv : {5, 6})
+                if (round_fill(cdiv(Nout, wv * per_wave)) > round_fill(cdiv(Nout, r->waves * per_wave)) + 0.02) r->waves = wv;
+    }
+    if (per <= 5 || per == 7 || (single && Mc <= 2) || (Mc == 1 && (per == 6 || per == 9 || per == 10 || (per == 8 && !whole))))
+        r->unroll = valu_depth(r->m_tiles, r->n_tiles, per);
+    else
+        r->unroll = per % 4 == 0 ? 4 : 2;
+}
+
+void lds_rule(int mt, int nt, int unroll, int kc, int channels, int splits, int x_preload, krk_gemm_config* r) {
+    r->kernel = KRK_KERNEL_MFMA_LDS;
+    r->m_tiles = mt;
+    r->n_tiles = nt;
+    r->unroll = unroll;
+    r->waves = krk::kLdsWaves;
+    r->splits = splits;
+    r->k_chunk = kc;
+    r->channels = channels;
+    r->x_preload = x_preload;
+}
+
+void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
+    const int mt = cdiv(Mc, 16);
+    const int KST = cdiv(K, 512);
+    const int Nout = silu ? N / 2 : N;
+    *c = krk_gemm_config{};
+    if (silu) {
+        if (Mc <= kValuMaxRows) return valu_rule(Mc, N, K, true, c);
+        // LDS-staged blocks of 24 or 32 channels, one per CU (4864 channels,
+        // K = 2560, M = 10 / 32 / 64: 13.4 / 14.5 / 17.2 against 19.0 / 20.3
+        // / 18.1 with 16-channel blocks or the stream kernel); up to 4096
+        // channels blocks of 16, with x in registers where its whole stages
+        // are the held ones, 5 or 8 (2432 channels, K = 2560, M = 16: 8.2
+        // against 17.4 with two splits; at 3 stages the zero stages cost
+        // more: 855 channels, K = 1088, M = 22: 8.9, 7.4 without), else K
+        // split while the blocks stay within one round (1500 channels, K =
+        // 5000, M = 32: 13.4 with 2 splits, 19.7 with 3, a second round).  Of
+        // 33 rows and more, few channels go to the stream kernel's blocks of
+        // 8 (268 channels, K = 1608, M = 37: 8.6 against 9.2), and so do more
+        // than one round holds while x fits its registers with K whole (12105
+        // channels, K = 1432, M = 39: 19.9 against 23.5).
+        if ((Mc > 32 && Nout <= 1200) || (Nout > 32 * kCuCount && K >= 1024 && stream_xs(mt, KST))) {
+            c->kernel = KRK_KERNEL_STREAM;
+            c->m_tiles = mt;
+            c->n_tiles = 1;
+            c->waves = krk::kStreamWaves;
+            c->unroll = mt <= 2 ? 5 : 4;
+            c->splits = 1;
+            while (c->splits < 32 && stream_xs(mt, cdiv(KST, c->splits)) == 0) ++c->splits;
+            return;
+        }
+        const int ch = even_channels(Nout, 32) <= 16 ? 16 : even_channels(Nout, 32);
+        const int nt = ch <= 16 ? 2 : 4;
+        const int kc = nt == 2 && mt <= 2 ? 512 : 256;
+        const int blocks = cdiv(Nout, ch);
+        const bool held = kc == 512 && (KST == krk::kLdsNormStages || (KST == krk::kLdsXpreStages && blocks >= kCuCount / 2));
+        int sp = 1;
+        if (!held)
+            while (blocks * (sp + 1) <= kCuCount && sp < 4 && KST >= 2 * (sp + 1)) ++sp;
+        lds_rule(mt, nt, mfma_lds_pf3(mt, nt) && KST > 3 && sp == 1 ? 3 : 2, kc, ch, sp, held ? 2 : 1, c);
+        return;
+    }
+    // Wave-sliced: 3-4 rows on few channels of a K that is long, or not whole
+    // blocks of the VALU kernel (M = 4, 2560 x 4864: 6.7 against 8.0, x 2432:
+    // 5.0 against 5.7; 3072 x 2560: 5.4 against 5.0), and
+    // 5-32 rows up to 32 channels per CU (3072 x 2560, M = 6 / 16 / 32: 5.5 /
+    // 6.2 / 7.5 against 8.5 / 9.4 / 10.0 with a split VALU or LDS-staged
+    // plan) unless both K and the channels are large, where the LDS-staged
+    // kernel takes x in longer runs (6810 x 7120, M = 16: 21.3 against 24.4),
+    // or K is long for 9-32 rows (400 x 9728, M = 32: 8.6 with 8 LDS-staged
+    // splits, over 10.8 here; 1984 x 9880, M = 15: 13.6 against 15.3).
+    const int per_cu = cdiv(N, kCuCount);
+    const bool few_rows = Mc >= 3 && Mc <= 4 && N <= 16 * kCuCount &&
+                          (K > 3072 || (K > 1024 && K % krk::kValuBlock != 0));
+    const bool sliced = Mc >= 5 && Mc <= 32 && per_cu <= kSliceMaxChannels && !(per_cu > 16 && K > 4096) &&
+                        !(Mc > 8 && K > 6656) &&
+                        !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 8 || per_cu > 12))));
+    const bool wide_sliced = Mc >= 5 && Mc <= 8 && per_cu > kSliceMaxChannels && K >= 2048 && K <= 8192;
+    if (few_rows || sliced || wide_sliced) {
+        c->kernel = KRK_KERNEL_SLICE;
+        c->unroll = 2;
+        c->waves = krk::kSliceWaves;
+        c->splits = 1;
+        // More channels than one round holds: 16 per block (37984 x 2560,
+        // M = 6: 31.4 against 33.3 on the stream kernel, 37.4 on the VALU).
+        c->channels = wide_sliced ? 16 : per_cu;
+        c->k_chunk = !wide_sliced && Mc <= 12 && c->channels <= 16 ? 128 : 64;
+        const SliceShape v = slice_shape(c->k_chunk, c->channels, Mc);
+        c->n_tiles = v.NT;
+        c->m_tiles = v.MT;
+        return;
+    }
+    if (Mc <= 4 || (Mc <= kValuMaxRows && per_cu > kSliceMaxChannels)) return valu_rule(Mc, N, K, false, c);
+    if (N >= 64 * kCuCount && K >= 1024 && stream_xs(mt, KST)) {
+        // A long weight stream and x that fits the registers with K whole
+        // (37984 x 2560, M = 10 / 32 / 64: 34.4 / 39.0 / 43.8 against 45.2 /
+        // 49.0 / 61.9 on 32-channel LDS-staged blocks).
+        c->kernel = KRK_KERNEL_STREAM;
+        c->m_tiles = mt;
+        c->n_tiles = 1;
+        c->waves = krk::kStreamWaves;
+        c->unroll = mt <= 2 ? 5 : 4;
+        c->splits = 1;
+        return;
+    }
+    if (N > 16 * kCuCount) {
+        // One round of blocks, or whole rounds of up to 64 channels (5120 x
+        // 3584, M = 48: 13.5 on 214 blocks of 24 channels, 22.4 on 2 splits
+        // of 160; 12288 x 4096: 23.4 against 33.2).  Three stages in flight
+        // up to three x tiles (6810 x 7120, M = 16: 21.3 against 23.9) unless
+        // K has few of them (6902 x 736, M = 50: 7.9, 7.1 with two).
+        const int ch = even_channels(N, 64);
+        const int nt = ch <= 32 ? 2 : 4;
+        const bool deep = mt <= 2 && nt == 2;
+        const bool three = mt <= 3 && mfma_lds_pf3(mt, nt) && K > 1536;
+        lds_rule(mt, nt, three ? 3 : 2, deep ? 512 : 256, ch, 1, 1, c);
+        return;
+    }
+    // Few channels.  A short K stays whole, on blocks of 16 or, below 2048
+    // channels, 8 (2560 x 2048, M = 48: 8.4 against 9.7 with 2 splits; 1536 x
+    // 2560: 8.6 against 10.2); a long K, or under 1024 channels, is split
+    // until the blocks fill the CUs, at least a stage and a half each (2560 x
+    // 4864, M = 64: 13.0 with 3 splits of 32 channels; 1938 x 7896, M = 57:
+    // 15.5 with 4 of 32, 18.0 with 2 of 16; 700 x 3000: 8.8 with 4 of 16, 10.4
+    // with 3 of 32; 400 x 9728: 9.4 with 8, 14.1 with 4 of 32).
+    if (K <= 3072 && N >= 1024) {
+        lds_rule(mt, 1, 3, 256, N < 2048 ? 8 : 16, 1, 1, c);
+        return;
+    }
+    if (KST <= 3) {
+        lds_rule(mt, 2, 2, 256, 32, 1, 1, c);
+        return;
+    }
+    const int nt = N >= 1024 ? 2 : 1;
+    const int blocks = cdiv(N, 16 * nt);
+    int sp = kCuCount / blocks < 8 ? kCuCount / blocks : 8;
+    if (sp > KST * 2 / 3) sp = KST * 2 / 3;
+    lds_rule(mt, nt, nt == 1 ? 3 : 2, mt + nt <= 4 && nt == 2 ? 512 : 256, 16 * nt, sp < 1 ? 1 : sp, 1, c);
+}
 
 // The plan of launches of up to 64 rows.
 void chunk_config(int Mc, int N, int K, int epilogue, krk_gemm_config* c) {
@@ -288,45 +510,7 @@ void chunk_config(int Mc, int N, int K, int epilogue, krk_gemm_config* c) {
             return;
         }
     }
-    // Other shapes.  M <= 8: the VALU row-streaming kernel, K split until
-    // about 600 workgroup-splits stream and the x slice fits LDS.  Larger M:
-    // the persistent stream kernel where x is large and the weight stream
-    // long (its x-in-registers design pays off), otherwise the LDS-staged
-    // MFMA kernel with K split until ~200 workgroups stream.
-    const int Nout = silu ? N / 2 : N;
-    krk_gemm_config r{};
-    r.m_tiles = mt;
-    if (Mc <= kValuMaxRows) {
-        r.kernel = KRK_KERNEL_VALU;
-        r.m_tiles = valu_mx(Mc);
-        r.n_tiles = (silu || Mc > 4) ? 2 : 1;
-        r.waves = 4;
-        const int nblocks = cdiv(Nout, r.waves * (silu ? r.n_tiles / 2 : r.n_tiles));
-        r.splits = 1;
-        while (r.splits < KST && r.splits < 32 &&
-               (nblocks * r.splits < 600 || krk::valu_lds_bytes(r.m_tiles, cdiv(KST, r.splits)) > kLdsBudget))
-            ++r.splits;
-        r.unroll = valu_depth(r.m_tiles, r.n_tiles, cdiv(KST, r.splits));
-    } else if (Mc > 32 && (silu || N >= 65536)) {
-        r.kernel = KRK_KERNEL_STREAM;
-        r.n_tiles = 1;
-        r.waves = 8;
-        r.unroll = 4;
-        r.splits = 1;
-        while (r.splits < 32 && stream_xs(mt, cdiv(KST, r.splits)) == 0) ++r.splits;
-    } else {
-        r.kernel = KRK_KERNEL_MFMA_LDS;
-        r.n_tiles = (N >= 65536 && Mc > 8) ? 4 : 2;
-        r.unroll = 2;
-        r.k_chunk = default_kc(mt, r.n_tiles);
-        r.waves = krk::kLdsWaves;
-        r.channels = 16 * (silu ? r.n_tiles / 2 : r.n_tiles);
-        r.x_preload = 1;
-        const int nblocks = cdiv(Nout, r.channels);
-        r.splits = 1;
-        while (nblocks * r.splits < 192 && r.splits < 4 && KST >= 2 * (r.splits + 1)) ++r.splits;
-    }
-    *c = r;
+    rule_config(Mc, N, K, silu, c);
 }
 
 // Splits of a plan for more than 64 rows: its workspace also holds the tile
@@ -345,10 +529,6 @@ void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
         ++c->splits;
 }
 
-// MFMA_LDS keeps `unroll` stages of row pieces in registers; three stages fit
-// 256 VGPRs without spilling up to this many 16-row tiles (m + n).
-constexpr int kLdsPf3MaxTiles = 6;
-constexpr bool mfma_lds_pf3(int MT, int NT) { return MT + NT <= kLdsPf3MaxTiles; }
 // MFMA_LDS with x held in registers for the whole K (x_preload = 2): 512-k
 // stages, K unsplit in at most kLdsXpreStages of them, up to two x tiles.
 constexpr int kLdsXpreMaxMTiles = 2;
@@ -356,10 +536,6 @@ inline bool lds_xpre_ok(const krk_gemm_config& c, int K) {
     const int most = c.m_tiles == 1 && c.n_tiles == 1 ? krk::kLdsXpreLongStages : krk::kLdsXpreStages;
     return c.k_chunk == 512 && c.splits == 1 && cdiv(K, 512) <= most && c.m_tiles <= kLdsXpreMaxMTiles;
 }
-
-// Dynamic LDS a gfx950 workgroup may use: 160 KB less room for the kernels'
-// static __shared__ variables.
-constexpr size_t kLdsMax = 163840 - kLdsReserve;
 
 // STREAM: x fragments live in 8·XS·MT VGPRs per lane; the instantiated XS
 // values per MT are the ones that stay within 256 VGPRs without spilling in

@@ -1,0 +1,52 @@
+"""The plan rule for shapes outside the dispatch table (host code only): every
+plan is one the library accepts as an explicit configuration and resolves to
+itself, and its split-K scratch fits the static scratch wherever one split's
+does many times over."""
+
+from __future__ import annotations
+
+import ctypes
+import random
+
+import pytest
+
+from kernels import _lib
+from kernels._lib import GemmConfig
+
+NONE, SILU = _lib.EPILOGUE_NONE, _lib.EPILOGUE_SILU_MUL
+
+
+def _shapes(seed, count):
+    rng = random.Random(seed)
+    for _ in range(count):
+        N = 2 * int(2 ** rng.uniform(0, 16))
+        K = 8 * int(2 ** rng.uniform(0, 11.5))
+        yield rng.choice([1, 2, 3, 4, 5, 8, 9, 12, 13, 16, 17, 24, 32, 33, 48, 49, 64, 65, 128, 200]), N, K
+
+
+@pytest.mark.parametrize("epi", [NONE, SILU])
+def test_plans_resolve_to_themselves(epi):
+    lib = _lib.load()
+    for M, N, K in _shapes(5 + epi, 4000):
+        plan, got = GemmConfig(), GemmConfig()
+        assert lib.krk_gemm_plan(M, N, K, epi, ctypes.byref(plan)) == 0
+        rc = lib.krk_gemm_resolve(M, N, K, epi, ctypes.byref(plan), ctypes.byref(got))
+        assert rc == 0, (M, N, K, plan.as_dict(), _lib.last_error())
+        assert got.as_dict() == plan.as_dict(), (M, N, K)
+        c = plan.as_dict()
+        ws = lib.krk_gemm_workspace_bytes(M, N, K, epi)
+        assert (ws > 0) == (c["splits"] > 1), (M, N, K, c)
+        assert c["splits"] <= max(1, -(-K // 256)), (M, N, K, c)
+
+
+def test_split_scratch_stays_small():
+    """The rule splits only narrow shapes: partial sums of at most 4 MB less
+    the counters, so the allocation-free call takes every plan but the VALU
+    kernel's for an x slice that fills LDS."""
+    lib = _lib.load()
+    for M, N, K in _shapes(11, 4000):
+        plan = GemmConfig()
+        assert lib.krk_gemm_plan(M, N, K, NONE, ctypes.byref(plan)) == 0
+        c = plan.as_dict()
+        if c["splits"] > 1 and not (c["kernel"] == _lib.KERNEL_VALU and c["m_tiles"] * K * 2 > 65536):
+            assert c["splits"] * min(M, 64) * N * 4 <= (4 << 20) - (64 << 10), (M, N, K, c)

@@ -1,0 +1,36 @@
+"""GPU parity of the plan rule for shapes outside the dispatch table, on both
+sides of each of its lines (rows, channels per CU, K) and at ragged sizes,
+against the oracle."""
+
+from __future__ import annotations
+
+import pytest
+
+from kernels import gemm as G
+from oracle import gemm_ref as R
+from test_gemm_gpu import check_gateup, check_linear
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 700, 3000), (1, 2562, 2504), (1, 4100, 4616), (2, 2050, 2560), (2, 300, 5640),   # VALU
+    (3, 515, 1032), (3, 4097, 1032), (4, 8201, 2048), (4, 2500, 3080), (8, 8300, 1000),  # VALU / wave-sliced
+    (5, 255, 72), (12, 4096, 1416), (13, 4104, 1416), (16, 8192, 520), (32, 8200, 520), (8, 8300, 2056),
+    (9, 600, 6672), (17, 1800, 4104), (24, 3300, 4104), (32, 500, 5128),                   # LDS-staged, split
+    (33, 1023, 1536), (33, 1024, 3072), (64, 2047, 2048), (48, 2048, 3080), (40, 5000, 1544), (64, 9000, 1528),
+    (16, 16390, 1024), (33, 16400, 1000),                                                  # stream
+])
+def test_rule_plans(device, M, N, K):
+    x, w = R.randn_bf16((M, K), 8100 + M + N), R.randn_bf16((N, K), 8200 + K, 0.02)
+    check_linear(x, w, f"rule {G.plan(M, N, K)}")
+
+
+@pytest.mark.parametrize("M,I,K", [
+    (1, 1025, 2824), (2, 300, 5640), (4, 2100, 1544), (6, 310, 4104), (8, 1201, 2560),     # VALU
+    (9, 4097, 520), (16, 300, 2560), (17, 2050, 4096), (32, 1300, 3600), (32, 500, 1800),  # LDS-staged
+    (33, 1200, 1000), (33, 1201, 1000), (64, 4500, 1032), (40, 8300, 1032),                # stream / LDS-staged
+])
+def test_rule_gateup_plans(device, M, I, K):
+    x, w = R.randn_bf16((M, K), 8300 + M + I), R.randn_bf16((2 * I, K), 8400 + K, 0.02)
+    check_gateup(x, w, f"rule {G.plan(M, 2 * I, K, 1)}")
