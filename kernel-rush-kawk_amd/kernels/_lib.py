@@ -118,6 +118,8 @@ _lock = threading.Lock()
 def load() -> ctypes.CDLL:
     """Load (once) and return the library.  Raises ImportError if it is not built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not LIB_PATH.exists():

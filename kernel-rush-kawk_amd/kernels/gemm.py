@@ -56,6 +56,40 @@ def normed_plan(M: int, N: int, K: int, epilogue: int = EPILOGUE_NONE) -> dict:
     return cfg.as_dict()
 
 
+# One eager call of a small projection is bound by the host (o_proj at M = 1: 5
+# us on the GPU, 11.5 us a call through the first form of these helpers, 7.6
+# now), so each property of an operand is read once, a passed check costs no
+# message, the stream comes as its raw handle and the device context is entered
+# only when another device is current.
+_BF16 = torch.bfloat16
+
+
+def _launch(fn, index: int, *args) -> None:
+    """``fn(*args, stream)`` on GPU ``index`` and torch's current stream there;
+    raises what the return code says."""
+    if index < 0:
+        raise ValueError("operands must be GPU tensors, got CPU tensors")
+    stream = torch._C._cuda_getCurrentRawStream(index)
+    if torch._C._cuda_getDevice() == index:
+        rc = fn(*args, stream)
+    else:
+        with torch.cuda.device(index):
+            rc = fn(*args, stream)
+    if rc:
+        _lib.check(rc)
+
+
+def _row_stride(name: str, t: torch.Tensor, rows: int | None, cols: int) -> int:
+    """The row stride of a [rows, cols] bf16 operand, checked."""
+    if isinstance(t, torch.Tensor) and t.dtype is _BF16 and t.dim() == 2:
+        r, c = t.shape
+        ld, one = t.stride()
+        if c == cols and one == 1 and (rows is None or r == rows):
+            return ld
+    _check_operand(name, t, rows, cols)
+    return t.stride(0)
+
+
 def _check_operand(name: str, t: torch.Tensor, rows: int | None, cols: int) -> None:
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch.Tensor")
@@ -78,14 +112,14 @@ def _check_norm(norm, M: int, K: int, device):
         d, wn, xout, eps = norm
     except (TypeError, ValueError):
         raise ValueError("norm must be a tuple (y, w_norm, xout, eps)") from None
-    _check_operand("norm y", d, M, K)
-    _check_operand("xout", xout, M, K)
-    if not isinstance(wn, torch.Tensor) or wn.dtype != torch.bfloat16 or wn.numel() != K or not wn.is_contiguous():
+    ldd = _row_stride("norm y", d, M, K)
+    ldxo = _row_stride("xout", xout, M, K)
+    if not isinstance(wn, torch.Tensor) or wn.dtype is not _BF16 or wn.numel() != K or not wn.is_contiguous():
         raise ValueError(f"w_norm must be a contiguous bf16 tensor of {K} elements")
     for name, t in (("norm y", d), ("w_norm", wn), ("xout", xout)):
         if t.device != device:
             raise ValueError(f"{name} must be on the operands' device {device}, got {t.device}")
-    return d, wn, xout, float(eps)
+    return d, ldd, wn, xout, ldxo, float(eps)
 
 
 def gemm_into(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, epilogue: int = EPILOGUE_NONE,
@@ -101,40 +135,31 @@ def gemm_into(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, epilogue: int =
     """
     M, K = x.shape
     N = w.shape[0]
-    _check_operand("x", x, None, K)
-    _check_operand("w", w, None, K)
-    nout = N // 2 if epilogue == EPILOGUE_SILU_MUL else N
-    _check_operand("y", y, M, nout)
-    for name, t in (("x", x), ("w", w), ("y", y)):
-        if t.device.type != "cuda":
-            raise ValueError(f"{name} must be a GPU tensor, got device {t.device}")
-    if not (x.device == w.device == y.device):
+    ldx = _row_stride("x", x, None, K)
+    ldw = _row_stride("w", w, None, K)
+    ldy = _row_stride("y", y, M, N // 2 if epilogue == EPILOGUE_SILU_MUL else N)
+    if not (x.is_cuda and w.is_cuda and y.is_cuda):
+        for name, t in (("x", x), ("w", w), ("y", y)):
+            if not t.is_cuda:
+                raise ValueError(f"{name} must be a GPU tensor, got device {t.device}")
+    index = x.get_device()
+    if not (index == w.get_device() == y.get_device()):
         raise ValueError(f"operands on different devices: {x.device}, {w.device}, {y.device}")
-    if norm is not None:
-        d, wn, xout, eps = _check_norm(norm, M, K, x.device)
     ws_ptr, ws_bytes = 0, 0
     if workspace is not None:
         if workspace.device != x.device:
             raise ValueError("workspace must be on the operands' device")
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
     lib = _lib.load()
-    cfg = GemmConfig.from_dict(config) if config is not None else None
-    with torch.cuda.device(x.device):
-        if norm is not None:
-            head = (x.data_ptr(), x.stride(0), d.data_ptr(), d.stride(0), wn.data_ptr(), eps, xout.data_ptr(),
-                    xout.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.stride(0), M, N, K, epilogue)
-            if cfg is None:
-                rc = lib.krk_gemm_bf16_normed(*head, ws_ptr, ws_bytes, stream)
-            else:
-                rc = lib.krk_gemm_bf16_normed_config(*head, ctypes.byref(cfg), ws_ptr, ws_bytes, stream)
-        elif cfg is None:
-            rc = lib.krk_gemm_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.stride(0),
-                                   M, N, K, epilogue, ws_ptr, ws_bytes, stream)
-        else:
-            rc = lib.krk_gemm_bf16_config(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
-                                          y.stride(0), M, N, K, epilogue, ctypes.byref(cfg), ws_ptr, ws_bytes, stream)
-    _lib.check(rc)
+    cfg = (ctypes.byref(GemmConfig.from_dict(config)),) if config is not None else ()
+    if norm is not None:
+        d, ldd, wn, xout, ldxo, eps = _check_norm(norm, M, K, x.device)
+        _launch(lib.krk_gemm_bf16_normed_config if cfg else lib.krk_gemm_bf16_normed, index,
+                x.data_ptr(), ldx, d.data_ptr(), ldd, wn.data_ptr(), eps, xout.data_ptr(), ldxo,
+                w.data_ptr(), ldw, y.data_ptr(), ldy, M, N, K, epilogue, *cfg, ws_ptr, ws_bytes)
+    else:
+        _launch(lib.krk_gemm_bf16_config if cfg else lib.krk_gemm_bf16, index,
+                x.data_ptr(), ldx, w.data_ptr(), ldw, y.data_ptr(), ldy, M, N, K, epilogue, *cfg, ws_ptr, ws_bytes)
     return y
 
 
@@ -147,16 +172,13 @@ def gemm_noalloc(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, epilogue: in
     time on one GPU share that scratch and must not be issued."""
     M, K = x.shape
     N = w.shape[0]
-    _check_operand("x", x, None, K)
-    _check_operand("w", w, None, K)
-    _check_operand("y", y, M, N // 2 if epilogue == EPILOGUE_SILU_MUL else N)
+    ldx = _row_stride("x", x, None, K)
+    ldw = _row_stride("w", w, None, K)
+    ldy = _row_stride("y", y, M, N // 2 if epilogue == EPILOGUE_SILU_MUL else N)
     if not (x.device == w.device == y.device) or x.device.type != "cuda":
         raise ValueError(f"operands must be on one GPU, got {x.device}, {w.device}, {y.device}")
-    with torch.cuda.device(x.device):
-        rc = _lib.load().krk_gemm_bf16_noalloc(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
-                                               y.stride(0), M, N, K, epilogue,
-                                               torch.cuda.current_stream(x.device).cuda_stream)
-    _lib.check(rc)
+    _launch(_lib.load().krk_gemm_bf16_noalloc, x.get_device(), x.data_ptr(), ldx, w.data_ptr(), ldw, y.data_ptr(), ldy,
+            M, N, K, epilogue)
     return y
 
 
@@ -188,16 +210,11 @@ def add_rms_norm(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: fl
     return ``rms_norm(xout, weight)`` — the reference's stand-alone kernel
     (engine/kernels/add_rmsnorm.py:32-43), on libkrk_gemm.so."""
     M, K = x.shape
-    _check_operand("x", x, None, K)
-    xo = x if xout is None else xout
-    d, wn, xo, eps = _check_norm((y, weight, xo, eps), M, K, x.device)
+    ldx = _row_stride("x", x, None, K)
+    d, ldd, wn, xo, ldxo, eps = _check_norm((y, weight, x if xout is None else xout, eps), M, K, x.device)
     out = torch.empty_like(x)
-    stream = torch.cuda.current_stream(x.device).cuda_stream
-    with torch.cuda.device(x.device):
-        rc = _lib.load().krk_add_rms_norm_bf16(x.data_ptr(), x.stride(0), d.data_ptr(), d.stride(0), wn.data_ptr(),
-                                               eps, xo.data_ptr(), xo.stride(0), out.data_ptr(), out.stride(0), M, K,
-                                               stream)
-    _lib.check(rc)
+    _launch(_lib.load().krk_add_rms_norm_bf16, x.get_device(), x.data_ptr(), ldx, d.data_ptr(), ldd, wn.data_ptr(), eps,
+            xo.data_ptr(), ldxo, out.data_ptr(), out.stride(0), M, K)
     return out
 
 
@@ -305,6 +322,7 @@ class SkinnyMatmul:
         if M < 1 or N < 1 or K < 8 or K % 8:
             raise ValueError(f"unsupported shape M={M} N={N} K={K} (need K >= 8, K % 8 == 0)")
         self.M, self.N, self.K = M, N, K
+        self._a_shape = (M, K)
         self.device = torch.device(device)
         triton_args = dict(block_n=block_n, block_k=block_k, split_k=split_k, num_warps=num_warps,
                            num_stages=num_stages)
@@ -324,7 +342,7 @@ class SkinnyMatmul:
 
     def run(self, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, norm=None) -> torch.Tensor:
         """Allocation-free form: write into ``out``."""
-        if a.shape[0] != self.M or a.shape[1] != self.K or w.shape[0] != self.N:
+        if a.shape != self._a_shape and (a.shape[0] != self.M or a.shape[1] != self.K) or w.shape[0] != self.N:
             raise ValueError(f"operands {tuple(a.shape)} x {tuple(w.shape)} do not match the "
                              f"({self.M}, {self.N}, {self.K}) this object was built for")
         return gemm_into(a, w, out, self.epilogue, self.workspace, self.config, norm)
@@ -332,7 +350,7 @@ class SkinnyMatmul:
     def __call__(self, a: torch.Tensor, w: torch.Tensor, norm=None) -> torch.Tensor:
         """``norm=(y, w_norm, xout, eps)`` fuses ``xout = a + y; a = rms_norm(xout, w_norm)``
         in front (reference signature, engine/kernels/gemm.py:346-347)."""
-        out = torch.empty((self.M, self.out_cols), dtype=torch.bfloat16, device=a.device)
+        out = torch.empty((self.M, self.out_cols), dtype=_BF16, device=a.device)
         return self.run(a, w, out, norm)
 
 
@@ -712,10 +730,8 @@ class SkinnySelect:
         the logits into ``logits`` ([M, N] bf16) and the selected values into
         ``values`` ([M, k] bf16)."""
         M, K, N, k = self.M, self.K, self.N, self.k
-        _check_operand("a", a, M, K)
-        _check_operand("w", w, N, K)
-        if logits is not None:
-            _check_operand("logits", logits, M, N)
+        lda, ldw = _row_stride("a", a, M, K), _row_stride("w", w, N, K)
+        ldy = N if logits is None else _row_stride("logits", logits, M, N)
         if idx.dtype != torch.int64 or tuple(idx.shape) != (M, k) or not idx.is_contiguous():
             raise ValueError(f"idx must be a contiguous int64 tensor of shape ({M}, {k})")
         if values is not None and (values.dtype != torch.bfloat16 or tuple(values.shape) != (M, k)
@@ -724,19 +740,15 @@ class SkinnySelect:
         for name, t in (("a", a), ("w", w), ("idx", idx), ("logits", logits), ("values", values)):
             if t is not None and t.device != self.device:
                 raise ValueError(f"{name} must be on {self.device}, got {t.device}")
-        stream = torch.cuda.current_stream(self.device).cuda_stream
         lib = _lib.load()
-        y_ptr, ldy = (logits.data_ptr(), logits.stride(0)) if logits is not None else (0, N)
-        v_ptr = values.data_ptr() if values is not None else 0
-        head = (a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), y_ptr, ldy, M, N, K, k, idx.data_ptr(), v_ptr)
+        head = (a.data_ptr(), lda, w.data_ptr(), ldw, 0 if logits is None else logits.data_ptr(), ldy, M, N, K, k,
+                idx.data_ptr(), 0 if values is None else values.data_ptr())
         ws = (self.workspace.data_ptr(), self.workspace.numel())
-        with torch.cuda.device(self.device):
-            if self.config is None:
-                rc = lib.krk_gemm_bf16_select(*head, *ws, stream)
-            else:
-                cfg = GemmConfig.from_dict(self.config)
-                rc = lib.krk_gemm_bf16_select_config(*head, ctypes.byref(cfg), *ws, stream)
-        _lib.check(rc)
+        if self.config is None:
+            _launch(lib.krk_gemm_bf16_select, idx.get_device(), *head, *ws)
+        else:
+            cfg = GemmConfig.from_dict(self.config)
+            _launch(lib.krk_gemm_bf16_select_config, idx.get_device(), *head, ctypes.byref(cfg), *ws)
         return idx
 
     def __call__(self, a: torch.Tensor, w: torch.Tensor, logits: torch.Tensor | None = None) -> torch.Tensor:
