@@ -157,7 +157,8 @@ typedef struct krk_gemm_config {
  * negative error for an invalid shape.  For more than 64 rows it describes the
  * launches of up to 64 rows; calls with it (or with no configuration) take
  * their larger launches on the tile kernel, whose own tiles follow from the
- * shape.  Any other configuration runs in launches of up to 64 rows.
+ * shape, and so do some shapes of 49 to 64 rows.  Any other configuration
+ * runs in launches of up to 64 rows on its own kernel.
  */
 int krk_gemm_plan(int M, int N, int K, int epilogue, krk_gemm_config* out);
 

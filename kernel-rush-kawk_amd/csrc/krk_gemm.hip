@@ -513,6 +513,24 @@ void chunk_config(int Mc, int N, int K, int epilogue, krk_gemm_config* c) {
     rule_config(Mc, N, K, silu, c);
 }
 
+// 49 to 64 rows that run on the tile kernel in place of the LDS-staged plan
+// (MI355X, graph replay over distinct weights, us): 65-80 plain or 33-40
+// SwiGLU channels per CU with K whole.  Five tiles hold them in one round of
+// blocks, the plan's four take two (16400 x 6144, M = 64: 60.8 -> 49.0;
+// x 520: 15.9 -> 11.0; 10000 SwiGLU channels, K = 3072: 37.4 -> 31.2).  At
+// four tiles and fewer both run one round and neither wins (14000 x 6144:
+// 41.1, 42.9 here; 8192 SwiGLU channels, K = 2560: 22.0, 22.6).  No split, so
+// no workspace.
+// At 48 rows and fewer the plan has three x tiles and wins or ties more often.
+constexpr int kTileMinRows = 49;
+bool tile_rows_ok(int M, int N, int epilogue, const krk_gemm_config& c) {
+    if (M < kTileMinRows || M > kMaxRowsPerLaunch || c.kernel != KRK_KERNEL_MFMA_LDS || c.splits > 1) return false;
+    const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
+    const int unit = silu ? 8 : 16;
+    const int per_cu = cdiv(silu ? N / 2 : N, kCuCount);
+    return per_cu > 4 * unit && per_cu <= krk::kTileMaxNT * unit;
+}
+
 // Splits of a plan for more than 64 rows: its workspace also holds the tile
 // kernel's partial sums, 128 rows x splits / 2 of them (tall_plan below).
 // Only plans that split K anyway take more splits, as many as the static
@@ -1054,7 +1072,7 @@ int dispatch_slice(const LaunchArgs& a, const krk_gemm_config& c, int nblocks, h
                             : dispatch_slice_kc<64>(a, v, c.unroll, nblocks, s);
 }
 
-// How one launch of the tile kernel cuts `rows` (65..128) rows: tiles, output
+// How one launch of the tile kernel cuts `rows` (49..128) rows: tiles, output
 // channels per block and K splits, whose partial sums fit part_bytes.
 struct TallPlan {
     int mt, nt, cb, splits, nblk;
@@ -1074,7 +1092,7 @@ TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
     const int stages = cdiv(K, krk::kTileKC);
     TallPlan best{};
     double best_us = 0.0;
-    const int mt = rows > 96 ? 8 : 6;
+    const int mt = rows > 96 ? 8 : rows > 64 ? 6 : 4;
     for (int sp = 1; sp <= krk::kTileMaxSplits && sp <= stages; ++sp) {
         // One block per CU and split, in the 4 channels of a store.
         const int64_t one = (((int64_t)Nout * sp + kCuCount - 1) / kCuCount + 3) / 4 * 4;
@@ -1126,13 +1144,16 @@ int dispatch_tile_n(const krk::TileArgs& a, int nt, hipStream_t s) {
     return fail(KRK_ERR_UNSUPPORTED, "tile kernel with %d weight tiles", nt);
 }
 
-// y of a.M (65..128) rows; part: part_bytes of workspace for split sums.
+// y of a.M (49..128) rows; part: part_bytes of workspace for split sums.
 int dispatch_tile(const LaunchArgs& a, int epilogue, size_t part_bytes, hipStream_t s) {
     const TallPlan p = tall_plan(a.M, a.N, a.K, epilogue, part_bytes);
     const krk::TileArgs t{a.x, a.ldx, a.w, a.ldw, a.y, a.ldy, a.M, a.N, a.K, p.splits, p.cb, p.nblk, a.part};
-    if (epilogue == KRK_EPILOGUE_SILU_MUL)
-        return p.mt == 8 ? dispatch_tile_n<8, true>(t, p.nt, s) : dispatch_tile_n<6, true>(t, p.nt, s);
-    return p.mt == 8 ? dispatch_tile_n<8, false>(t, p.nt, s) : dispatch_tile_n<6, false>(t, p.nt, s);
+    const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
+    switch (p.mt) {
+        case 4: return silu ? dispatch_tile_n<4, true>(t, p.nt, s) : dispatch_tile_n<4, false>(t, p.nt, s);
+        case 6: return silu ? dispatch_tile_n<6, true>(t, p.nt, s) : dispatch_tile_n<6, false>(t, p.nt, s);
+        default: return silu ? dispatch_tile_n<8, true>(t, p.nt, s) : dispatch_tile_n<8, false>(t, p.nt, s);
+    }
 }
 
 template <int MX, int R, int D, bool SILU, bool NORM = false, bool SEL = false>
@@ -1461,7 +1482,8 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     }
     // More than 64 rows under the plan (a configuration equal to it included):
     // launches of up to 128 rows on the tile kernel while more than 64 are left.
-    bool tall = M > kMaxRowsPerLaunch && !fused;
+    // 49 to 64 rows: one launch of it where tile_rows_ok says so.
+    bool tall = !fused && (M > kMaxRowsPerLaunch || tile_rows_ok(M, N, epilogue, c));
     if (tall) {
         krk_gemm_config plan;
         auto_config(M, N, K, epilogue, &plan);
@@ -1470,7 +1492,7 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     }
     int rows = 0;
     for (int m0 = 0; m0 < M; m0 += rows) {
-        const bool tile = tall && M - m0 > kMaxRowsPerLaunch;
+        const bool tile = tall && (M - m0 > kMaxRowsPerLaunch || M <= kMaxRowsPerLaunch);
         const int most = tile ? krk::kTileMaxRows : kMaxRowsPerLaunch;
         rows = M - m0 < most ? M - m0 : most;
         LaunchArgs a;

@@ -1,6 +1,7 @@
 // Tall-tile MFMA skinny GEMM (gfx950): y = epilogue(x[M,K] · W[N,K]ᵀ) for 65
 // to 128 rows in one launch, so that a batch of more than 64 rows reads W
-// once instead of once per 64 rows.
+// once instead of once per 64 rows; and for 49 to 64 rows of the shapes that
+// it is faster on (tile_rows_ok, with the figures).
 //
 // Reference counterparts: _skinny_kernel / _gateup_kernel with split-K and
 // their sum kernels (engine/kernels/gemm.py:54-104, 116-170); the reference

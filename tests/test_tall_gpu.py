@@ -38,6 +38,17 @@ def test_gateup_rows_beyond_64(device, M, I, K):
     check_gateup(x, wgu, f"tall gateup M={M} I={I} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K,epi", [
+    (49, 16385, 72, NONE), (64, 20480, 520, NONE), (63, 18000, 2568, NONE),
+    (49, 2 * 8193, 136, SILU), (64, 2 * 10240, 264, SILU), (60, 2 * 9001, 2632, SILU),
+])
+def test_49_to_64_rows(device, M, N, K, epi):
+    """The shapes that run on the tile kernel below 65 rows, at the ends of
+    their ranges."""
+    x, w = R.randn_bf16((M, K), 9250 + M), R.randn_bf16((N, K), 9350 + N, 0.02)
+    (check_gateup if epi == SILU else check_linear)(x, w, f"tile M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("M,N,K,ypad", [(100, 77, 520, 3), (128, 2560, 1024, 4), (70, 64, 264, 1)])
 def test_strided_operands(device, M, N, K, ypad):
     """Row strides past the operands' widths; y with rows that are not 8-byte
