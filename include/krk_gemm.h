@@ -94,7 +94,8 @@ size_t krk_gemm_workspace_bytes(int M, int N, int K, int epilogue);
  * Kernel configuration.  Mirrors the per-candidate config dicts of the
  * reference (engine/kernels/gemm.py:284-288 GEMV_CONFIGS, :364-375 CONFIGS)
  * that SkinnyMatmul/Gemv are constructed from (gemm.py:251, 301, 333).
- * A field left at 0 takes the dispatcher's choice for this shape.
+ * A field left at 0 takes the dispatcher's choice for this shape: the plan's
+ * value, or where that does not go with the fields given, another that does.
  */
 enum {
     KRK_KERNEL_AUTO = 0,
@@ -178,14 +179,14 @@ int krk_gemm_candidates(int M, int N, int K, int epilogue, krk_gemm_config* out,
 
 /*
  * krk_gemm_config_workspace_bytes — as krk_gemm_workspace_bytes, for an
- * explicit configuration (0 fields filled from krk_gemm_plan).
+ * explicit configuration (0 fields filled as krk_gemm_config says).
  */
 size_t krk_gemm_config_workspace_bytes(int M, int N, int K, int epilogue,
                                        const krk_gemm_config* cfg);
 
 /*
  * krk_gemm_resolve — the configuration krk_gemm_bf16_config runs for `cfg`
- * (0 fields filled from krk_gemm_plan; NULL = the plan itself), or
+ * (0 fields filled as krk_gemm_config says; NULL = the plan itself), or
  * KRK_ERR_UNSUPPORTED / KRK_ERR_INVALID with krk_last_error() explaining why
  * this build cannot run it.  The check the reference's constructors make
  * before a launch (SkinnyMatmul / SkinnyGateUp / Gemv.__init__,

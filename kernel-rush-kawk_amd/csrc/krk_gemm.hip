@@ -589,12 +589,47 @@ inline int stream_groups(int nblocks, int splits) {
     return best;
 }
 
-// Fill the zero fields of a caller's configuration from the table and check
-// that the result is one this build instantiates.
-int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in, krk_gemm_config* out) {
-    krk_gemm_config a;
-    auto_config(M, N, K, epilogue, &a);
-    if (!in) { *out = a; return KRK_OK; }
+// What a partial configuration is completed from where the plan's fields do
+// not go with the caller's (its kernel, tiles or K chunks are others): the
+// fields of this simpler rule combine with more of them.  M <= 8: VALU, K split
+// until about 600 blocks run and the x slice fits 64 KB of LDS; more than 32
+// rows with SwiGLU or many channels: stream; else LDS-staged, K split until
+// about 200 blocks run.
+void filler_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
+    const int mt = cdiv(Mc, 16), KST = cdiv(K, 512), Nout = silu ? N / 2 : N;
+    krk_gemm_config r{};
+    r.m_tiles = mt;
+    r.splits = 1;
+    if (Mc <= kValuMaxRows) {
+        r.kernel = KRK_KERNEL_VALU;
+        r.m_tiles = valu_mx(Mc);
+        r.n_tiles = silu || Mc > 4 ? 2 : 1;
+        r.waves = 4;
+        const int blocks = cdiv(Nout, silu ? 4 : 4 * r.n_tiles);
+        while (r.splits < KST && r.splits < 32 &&
+               (blocks * r.splits < 600 || krk::valu_lds_bytes(r.m_tiles, cdiv(KST, r.splits)) > kLdsBudget))
+            ++r.splits;
+        r.unroll = valu_depth(r.m_tiles, r.n_tiles, cdiv(KST, r.splits));
+    } else if (Mc > 32 && (silu || N >= 65536)) {
+        r.kernel = KRK_KERNEL_STREAM;
+        r.n_tiles = 1;
+        r.waves = krk::kStreamWaves;
+        r.unroll = 4;
+        while (r.splits < 32 && stream_xs(mt, cdiv(KST, r.splits)) == 0) ++r.splits;
+    } else {
+        const int nt = N >= 65536 && Mc > 8 ? 4 : 2;
+        const int channels = 16 * (silu ? nt / 2 : nt);
+        int sp = 1;
+        while (cdiv(Nout, channels) * sp < 192 && sp < 4 && KST >= 2 * (sp + 1)) ++sp;
+        lds_rule(mt, nt, 2, default_kc(mt, nt), channels, sp, 1, &r);
+    }
+    *c = r;
+}
+
+// Fill the zero fields of a caller's configuration from `a` and check that
+// the result is one this build instantiates.
+int complete_config(int M, int N, int K, int epilogue, const krk_gemm_config& a, const krk_gemm_config* in,
+                    krk_gemm_config* out) {
     krk_gemm_config c = *in;
     if (c.prologue != 0 && c.prologue != 1)
         return fail(KRK_ERR_UNSUPPORTED, "prologue=%d not in {0, 1}", c.prologue);
@@ -745,6 +780,23 @@ int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in,
         return fail(KRK_ERR_UNSUPPORTED, "splits=%d not in 1..32", c.splits);
     *out = c;
     return KRK_OK;
+}
+
+// A caller's configuration with its zero fields filled from the plan, or
+// where that is none this build runs, from filler_config.
+int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in, krk_gemm_config* out) {
+    krk_gemm_config a;
+    auto_config(M, N, K, epilogue, &a);
+    if (!in) { *out = a; return KRK_OK; }
+    const int rc = complete_config(M, N, K, epilogue, a, in, out);
+    if (rc == KRK_OK) return rc;
+    krk_gemm_config f;
+    filler_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue == KRK_EPILOGUE_SILU_MUL, &f);
+    if (complete_config(M, N, K, epilogue, f, in, out) == KRK_OK) {
+        g_err[0] = '\0';
+        return KRK_OK;
+    }
+    return complete_config(M, N, K, epilogue, a, in, out);  // the reason against the plan's fields
 }
 
 // Workspace layout: [block counters, padded to 256 B][fp32 partials splits x Mc x N].

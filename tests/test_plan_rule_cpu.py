@@ -39,6 +39,29 @@ def test_plans_resolve_to_themselves(epi):
         assert c["splits"] <= max(1, -(-K // 256)), (M, N, K, c)
 
 
+@pytest.mark.parametrize("M,N,K,epi,cfg", [
+    (64, 10106, 8192, SILU, {"kernel": _lib.KERNEL_STREAM}),           # the plan is LDS-staged with K whole
+    (200, 96224, 14336, NONE, {"kernel": _lib.KERNEL_STREAM, "unroll": 2}),
+    (200, 96224, 14336, SILU, {"kernel": _lib.KERNEL_MFMA_LDS, "unroll": 3}),   # the plan has four weight tiles
+    (13, 58940, 8192, SILU, {"kernel": _lib.KERNEL_MFMA_LDS, "k_chunk": 512, "m_tiles": 2}),
+    (33, 73576, 992, NONE, {"kernel": _lib.KERNEL_MFMA_LDS, "k_chunk": 512, "splits": 4}),
+    (12, 21042, 9728, SILU, {"channels": 8, "k_chunk": 512}),
+    (12, 300, 88, NONE, {"k_chunk": 256}),                             # the plan is wave-sliced
+    (4, 20, 4096, NONE, {"unroll": 5}),
+    (128, 80648, 14336, SILU, {"unroll": 7, "splits": 7}),
+])
+def test_partial_configurations_are_completed(M, N, K, epi, cfg):
+    """A configuration that names only some fields runs where some choice of
+    the others does, whatever the plan's are, and keeps the named ones."""
+    lib = _lib.load()
+    given, got, again = GemmConfig.from_dict(cfg), GemmConfig(), GemmConfig()
+    assert lib.krk_gemm_resolve(M, N, K, epi, ctypes.byref(given), ctypes.byref(got)) == 0, _lib.last_error()
+    out = got.as_dict()
+    assert {k: out[k] for k in cfg} == cfg
+    assert lib.krk_gemm_resolve(M, N, K, epi, ctypes.byref(got), ctypes.byref(again)) == 0
+    assert again.as_dict() == out
+
+
 def test_split_scratch_stays_small():
     """The rule splits only narrow shapes: partial sums of at most 4 MB less
     the counters, so the allocation-free call takes every plan but the VALU
