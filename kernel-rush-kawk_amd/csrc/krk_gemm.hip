@@ -531,20 +531,70 @@ bool tile_rows_ok(int M, int N, int epilogue, const krk_gemm_config& c) {
     return per_cu > 4 * unit && per_cu <= krk::kTileMaxNT * unit;
 }
 
-// Splits of a plan for more than 64 rows: its workspace also holds the tile
-// kernel's partial sums, 128 rows x splits / 2 of them (tall_plan below).
-// Only plans that split K anyway take more splits, as many as the static
-// scratch of krk_gemm_bf16_noalloc holds; the block counters keep their place
-// (the block geometry does not change).
-constexpr int kTallPlanSplits = 6;
-
 void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
     chunk_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue, c);
-    if (M <= kMaxRowsPerLaunch || c->kernel != KRK_KERNEL_MFMA_LDS || c->splits == 1) return;
-    const size_t one = (size_t)kMaxRowsPerLaunch * N * sizeof(float);
-    while (c->splits < kTallPlanSplits && c->splits < cdiv(K, 512) &&
-           (c->splits + 1) * one <= KRK_NOALLOC_SCRATCH_BYTES - KRK_NOALLOC_COUNTER_BYTES)
-        ++c->splits;
+}
+
+// How one launch of the tile kernel cuts `rows` (49..128) rows: tiles, output
+// channels per block and K splits, whose partial sums fit part_bytes.
+struct TallPlan {
+    int mt, nt, cb, splits, nblk;
+};
+
+// The cheapest cut under a linear model of the measured times (MI355X, 96 and
+// 128 rows of the Qwen3-4B projections): a CU takes in 47 KB of x and W
+// together per us, a launch costs 3 us beside that, and a split K the second
+// launch's 4 us.  The model puts qkv, gate_up and lm_head on whole K (qkv
+// M = 128: 17.0 us against 18.4 with 2 splits) and o and down on the most
+// splits their workspace holds (o: 16.2 with 4 splits, 24 unsplit).  Blocks
+// are cut to one per CU where the tiles allow it.
+TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
+    const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
+    const int Nout = silu ? N / 2 : N;
+    const int unit = silu ? 8 : 16;  // output channels of a W tile
+    const int stages = cdiv(K, krk::kTileKC);
+    TallPlan best{};
+    double best_us = 0.0;
+    const int mt = rows > 96 ? 8 : rows > 64 ? 6 : 4;
+    for (int sp = 1; sp <= krk::kTileMaxSplits && sp <= stages; ++sp) {
+        // One block per CU and split, in the 4 channels of a store.
+        const int64_t one = (((int64_t)Nout * sp + kCuCount - 1) / kCuCount + 3) / 4 * 4;
+        for (int nt = 2; nt <= krk::kTileMaxNT; ++nt)
+            for (int cb : {(int)(one < nt * unit ? one : nt * unit), nt * unit}) {
+                if (nt > 2 && cb <= (nt - 1) * unit) continue;  // fewer tiles hold it
+                TallPlan p{mt, nt, cb, sp, cdiv(Nout, cb)};
+                if (sp > 1 && sp * krk::tile_part_bytes(mt, nt, p.nblk) > part_bytes) continue;
+                const double bytes = 16.0 * (mt + nt) * 2 * krk::kTileKC * cdiv(stages, sp);
+                const double us = 3.0 + cdiv(p.nblk * sp, kCuCount) * bytes / 47e3 + (sp > 1 ? 4.0 : 0.0);
+                if (!best.mt || us < best_us) {
+                    best = p;
+                    best_us = us;
+                }
+            }
+    }
+    return best;
+}
+
+// Partial sums of the tile kernel's launches in a call of M > 64 rows whose
+// plan is c: at most what the static scratch of krk_gemm_bf16_noalloc holds,
+// so that every form of a call cuts K alike, and none where the plan keeps K
+// whole, whose calls bring no workspace.
+constexpr size_t kTallPartMax = KRK_NOALLOC_SCRATCH_BYTES - KRK_NOALLOC_COUNTER_BYTES;
+inline TallPlan tall_cut(int rows, int N, int K, int epilogue, const krk_gemm_config& c) {
+    return tall_plan(rows, N, K, epilogue, c.splits > 1 ? kTallPartMax : 0);
+}
+size_t tall_part(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
+    size_t most = 0;
+    const int last = M % krk::kTileMaxRows;  // of the launches of 128 rows
+    for (int rows : {M < krk::kTileMaxRows ? M : krk::kTileMaxRows, last}) {
+        if (rows <= kMaxRowsPerLaunch) continue;
+        const TallPlan p = tall_cut(rows, N, K, epilogue, c);
+        if (p.splits > 1) {
+            const size_t bytes = p.splits * krk::tile_part_bytes(p.mt, p.nt, p.nblk);
+            if (bytes > most) most = bytes;
+        }
+    }
+    return most;
 }
 
 // MFMA_LDS with x held in registers for the whole K (x_preload = 2): 512-k
@@ -799,12 +849,28 @@ int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in,
     return complete_config(M, N, K, epilogue, a, in, out);  // the reason against the plan's fields
 }
 
-// Workspace layout: [block counters, padded to 256 B][fp32 partials splits x Mc x N].
-size_t workspace_for(int M, int N, int epilogue, const krk_gemm_config& c) {
+// Whether a call with configuration c takes launches on the tile kernel: the
+// plan (a configuration equal to it included) at more than 64 rows, and at 49
+// to 64 where tile_rows_ok says so.
+bool tall_call(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
+    if (M <= kMaxRowsPerLaunch && !tile_rows_ok(M, N, epilogue, c)) return false;
+    krk_gemm_config plan;
+    auto_config(M, N, K, epilogue, &plan);
+    plan.prologue = c.prologue;
+    return !memcmp(&plan, &c, sizeof c);
+}
+
+// Workspace layout: [block counters, padded to 256 B][fp32 partials: splits x
+// Mc x N, or the tile kernel's where they are more].
+size_t workspace_for(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
     if (c.splits <= 1) return 0;
     const Geometry g = geometry(M, N, epilogue, c);
-    return align_up((size_t)g.nblocks * sizeof(uint32_t), 256) +
-           (size_t)c.splits * (size_t)g.Mc * (size_t)N * sizeof(float);
+    size_t part = (size_t)c.splits * (size_t)g.Mc * (size_t)N * sizeof(float);
+    if (M > kMaxRowsPerLaunch && tall_call(M, N, K, epilogue, c)) {
+        const size_t tall = tall_part(M, N, K, epilogue, c);
+        if (tall > part) part = tall;
+    }
+    return align_up((size_t)g.nblocks * sizeof(uint32_t), 256) + part;
 }
 
 bool overlaps(uintptr_t a0, uintptr_t a1, uintptr_t b0, uintptr_t b1) { return a0 < b1 && b0 < a1; }
@@ -1124,46 +1190,6 @@ int dispatch_slice(const LaunchArgs& a, const krk_gemm_config& c, int nblocks, h
                             : dispatch_slice_kc<64>(a, v, c.unroll, nblocks, s);
 }
 
-// How one launch of the tile kernel cuts `rows` (49..128) rows: tiles, output
-// channels per block and K splits, whose partial sums fit part_bytes.
-struct TallPlan {
-    int mt, nt, cb, splits, nblk;
-};
-
-// The cheapest cut under a linear model of the measured times (MI355X, 96 and
-// 128 rows of the Qwen3-4B projections): a CU takes in 47 KB of x and W
-// together per us, a launch costs 3 us beside that, and a split K the second
-// launch's 4 us.  The model puts qkv, gate_up and lm_head on whole K (qkv
-// M = 128: 17.0 us against 18.4 with 2 splits) and o and down on the most
-// splits their workspace holds (o: 16.2 with 4 splits, 24 unsplit).  Blocks
-// are cut to one per CU where the tiles allow it.
-TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
-    const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
-    const int Nout = silu ? N / 2 : N;
-    const int unit = silu ? 8 : 16;  // output channels of a W tile
-    const int stages = cdiv(K, krk::kTileKC);
-    TallPlan best{};
-    double best_us = 0.0;
-    const int mt = rows > 96 ? 8 : rows > 64 ? 6 : 4;
-    for (int sp = 1; sp <= krk::kTileMaxSplits && sp <= stages; ++sp) {
-        // One block per CU and split, in the 4 channels of a store.
-        const int64_t one = (((int64_t)Nout * sp + kCuCount - 1) / kCuCount + 3) / 4 * 4;
-        for (int nt = 2; nt <= krk::kTileMaxNT; ++nt)
-            for (int cb : {(int)(one < nt * unit ? one : nt * unit), nt * unit}) {
-                if (nt > 2 && cb <= (nt - 1) * unit) continue;  // fewer tiles hold it
-                TallPlan p{mt, nt, cb, sp, cdiv(Nout, cb)};
-                if (sp > 1 && sp * krk::tile_part_bytes(mt, nt, p.nblk) > part_bytes) continue;
-                const double bytes = 16.0 * (mt + nt) * 2 * krk::kTileKC * cdiv(stages, sp);
-                const double us = 3.0 + cdiv(p.nblk * sp, kCuCount) * bytes / 47e3 + (sp > 1 ? 4.0 : 0.0);
-                if (!best.mt || us < best_us) {
-                    best = p;
-                    best_us = us;
-                }
-            }
-    }
-    return best;
-}
-
 template <int MT, int NT, bool SILU>
 int launch_tile(const krk::TileArgs& a, hipStream_t stream) {
     constexpr int D = krk::tile_depth(MT, NT, kLdsMax);
@@ -1196,9 +1222,8 @@ int dispatch_tile_n(const krk::TileArgs& a, int nt, hipStream_t s) {
     return fail(KRK_ERR_UNSUPPORTED, "tile kernel with %d weight tiles", nt);
 }
 
-// y of a.M (49..128) rows; part: part_bytes of workspace for split sums.
-int dispatch_tile(const LaunchArgs& a, int epilogue, size_t part_bytes, hipStream_t s) {
-    const TallPlan p = tall_plan(a.M, a.N, a.K, epilogue, part_bytes);
+// y of a.M (49..128) rows, cut as p; part holds its split sums.
+int dispatch_tile(const LaunchArgs& a, int epilogue, const TallPlan& p, hipStream_t s) {
     const krk::TileArgs t{a.x, a.ldx, a.w, a.ldw, a.y, a.ldy, a.M, a.N, a.K, p.splits, p.cb, p.nblk, a.part};
     const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
     switch (p.mt) {
@@ -1421,7 +1446,7 @@ struct WorkspaceLayout {
 };
 WorkspaceLayout workspace_layout(int M, int N, int K, int epilogue, const krk_gemm_config& c, bool normed) {
     WorkspaceLayout l;
-    l.gemm = workspace_for(M, N, epilogue, c);
+    l.gemm = workspace_for(M, N, K, epilogue, c);
     const bool prologue = normed && !norm_fused(M, N, K, epilogue, c);
     const size_t nbytes = frag_prologue(M, c) ? krk::frag_bytes(c.m_tiles, K) : (size_t)M * K * sizeof(uint16_t);
     l.n_off = prologue ? align_up(l.gemm, 256) : 0;
@@ -1535,13 +1560,7 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     // More than 64 rows under the plan (a configuration equal to it included):
     // launches of up to 128 rows on the tile kernel while more than 64 are left.
     // 49 to 64 rows: one launch of it where tile_rows_ok says so.
-    bool tall = !fused && (M > kMaxRowsPerLaunch || tile_rows_ok(M, N, epilogue, c));
-    if (tall) {
-        krk_gemm_config plan;
-        auto_config(M, N, K, epilogue, &plan);
-        plan.prologue = c.prologue;
-        tall = !memcmp(&plan, &c, sizeof c);
-    }
+    const bool tall = !fused && tall_call(M, N, K, epilogue, c);
     int rows = 0;
     for (int m0 = 0; m0 < M; m0 += rows) {
         const bool tile = tall && (M - m0 > kMaxRowsPerLaunch || M <= kMaxRowsPerLaunch);
@@ -1562,7 +1581,7 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
         a.ctr = ctr;
         a.cb = g.cb;
         if (tile) {
-            rc = dispatch_tile(a, epilogue, part ? (size_t)c.splits * kMaxRowsPerLaunch * N * sizeof(float) : 0, st);
+            rc = dispatch_tile(a, epilogue, tall_cut(rows, N, K, epilogue, c), st);
         } else if (fused) {
             // This chunk's rows of d and xout.
             krk::NormArgs nc = na;
@@ -1679,11 +1698,11 @@ struct SelectLayout {
     int n;       // source elements per row
     int chunks;  // select_rows_kernel chunks per row
 };
-SelectLayout select_layout(int M, int N, int k, const SelectPlan& p) {
+SelectLayout select_layout(int M, int N, int K, int k, const SelectPlan& p) {
     const int Mc = M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch;
     SelectLayout l;
     l.proj = (size_t)krk::kSelMaxRows * krk::kSelCtrStride * sizeof(uint32_t);
-    size_t at = align_up(l.proj + workspace_for(Mc, N, KRK_EPILOGUE_NONE, p.c), 256);
+    size_t at = align_up(l.proj + workspace_for(Mc, N, K, KRK_EPILOGUE_NONE, p.c), 256);
     l.src = at;
     if (p.fused) {
         // One key per row and projection workgroup (the stream kernel's
@@ -1728,7 +1747,7 @@ int select_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y,
     if (y && ldy < N) return fail(KRK_ERR_INVALID, "ldy=%lld must be >= N=%d", (long long)ldy, N);
     SelectPlan p;
     if ((rc = select_plan_for(M, N, K, k, cfg, &p))) return rc;
-    const SelectLayout l = select_layout(M, N, k, p);
+    const SelectLayout l = select_layout(M, N, K, k, p);
 
     const uintptr_t x0 = (uintptr_t)x, x1 = x0 + ((uint64_t)(M - 1) * ldx + K) * 2;
     const uintptr_t w0 = (uintptr_t)w, w1 = w0 + ((uint64_t)(N - 1) * ldw + K) * 2;
@@ -1971,7 +1990,7 @@ size_t krk_gemm_select_workspace_bytes(int M, int N, int K, int k, const krk_gem
     if (check_shape(M, N, K, KRK_EPILOGUE_NONE) || k < 1 || k > krk::kSelMaxK || k > N) return 0;
     SelectPlan p;
     if (select_plan_for(M, N, K, k, cfg, &p)) return 0;
-    return select_layout(M, N, k, p).total;
+    return select_layout(M, N, K, k, p).total;
 }
 
 int krk_gemm_select_plan(int M, int N, int K, int k, krk_gemm_config* out) {
@@ -2025,14 +2044,14 @@ size_t krk_gemm_workspace_bytes(int M, int N, int K, int epilogue) {
     if (check_shape(M, N, K, epilogue)) return 0;
     krk_gemm_config c;
     auto_config(M, N, K, epilogue, &c);
-    return workspace_for(M, N, epilogue, c);
+    return workspace_for(M, N, K, epilogue, c);
 }
 
 size_t krk_gemm_config_workspace_bytes(int M, int N, int K, int epilogue, const krk_gemm_config* cfg) {
     if (check_shape(M, N, K, epilogue)) return 0;
     krk_gemm_config c;
     if (resolve_config(M, N, K, epilogue, cfg, &c)) return 0;
-    return workspace_for(M, N, epilogue, c);
+    return workspace_for(M, N, K, epilogue, c);
 }
 
 int krk_gemm_resolve(int M, int N, int K, int epilogue, const krk_gemm_config* cfg, krk_gemm_config* out) {

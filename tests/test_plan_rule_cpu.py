@@ -62,6 +62,27 @@ def test_partial_configurations_are_completed(M, N, K, epi, cfg):
     assert again.as_dict() == out
 
 
+def test_plans_beyond_64_rows_are_the_64_row_plans():
+    """A call of more than 64 rows runs its last launch, of up to 64, on the
+    64-row plan, K splits included; what the larger launches need on top only
+    shows in the workspace, which stays within the static scratch."""
+    lib = _lib.load()
+    shapes = [(130, 2560, 4096), (192, 2560, 9728), (66, 1938, 7896)] + list(_shapes(17, 2000))
+    for M, N, K in shapes:
+        M = 65 + M % 192
+        for epi in (NONE, SILU):
+            plan, base = GemmConfig(), GemmConfig()
+            assert lib.krk_gemm_plan(M, N, K, epi, ctypes.byref(plan)) == 0
+            assert lib.krk_gemm_plan(64, N, K, epi, ctypes.byref(base)) == 0
+            assert plan.as_dict() == base.as_dict(), (M, N, K, epi)
+            need, need64 = lib.krk_gemm_workspace_bytes(M, N, K, epi), lib.krk_gemm_workspace_bytes(64, N, K, epi)
+            assert need64 <= need <= max(need64, 4 << 20), (M, N, K, epi)
+        if N >= 8:
+            assert lib.krk_gemm_select_plan(M, N, K, 8, ctypes.byref(plan)) == 0
+            assert lib.krk_gemm_select_plan(64, N, K, 8, ctypes.byref(base)) == 0
+            assert plan.as_dict() == base.as_dict(), (M, N, K, "select")
+
+
 def test_split_scratch_stays_small():
     """The rule splits only narrow shapes: partial sums of at most 4 MB less
     the counters, so the allocation-free call takes every plan but the VALU

@@ -24,6 +24,7 @@ NONE, SILU = _lib.EPILOGUE_NONE, _lib.EPILOGUE_SILU_MUL
 @pytest.mark.parametrize("M,N,K", [
     (65, 96, 2560), (80, 250, 520), (96, 33, 136), (97, 2560, 4096), (128, 2560, 1416), (112, 6144, 264),
     (66, 40, 72), (128, 3, 8), (129, 100, 1000), (193, 18, 2568), (256, 21000, 128), (128, 2560, 9728),
+    (104, 70, 9728), (128, 400, 9728), (97, 3500, 4104), (130, 1938, 7896),   # K splits of few channels
 ])
 def test_rows_beyond_64(device, M, N, K):
     x = R.randn_bf16((M, K), 9100 + M)
@@ -31,7 +32,8 @@ def test_rows_beyond_64(device, M, N, K):
     check_linear(x, w, f"tall M={M} N={N} K={K}")
 
 
-@pytest.mark.parametrize("M,I,K", [(65, 24, 2560), (96, 1, 40), (97, 333, 1000), (128, 1216, 2560), (130, 70, 136)])
+@pytest.mark.parametrize("M,I,K", [(65, 24, 2560), (96, 1, 40), (97, 333, 1000), (128, 1216, 2560), (130, 70, 136),
+                                   (65, 33, 6144), (120, 307, 9600), (97, 2017, 4104)])  # K splits of few channels
 def test_gateup_rows_beyond_64(device, M, I, K):
     x = R.randn_bf16((M, K), 9300 + M)
     wgu = R.randn_bf16((2 * I, K), 9400 + I, 0.02)
@@ -98,11 +100,13 @@ def test_normed_rows_beyond_64(device):
     assert_parity(y.cpu(), ref, "normed")
 
 
-@pytest.mark.parametrize("M", [96, 128, 200])
+@pytest.mark.parametrize("M", [96, 128, 130, 192, 200])
 def test_forms_of_the_call_agree(device, M):
     """A split plan (o_proj): repeated calls, the allocation-free call and the
-    plan given as a configuration are bit-identical, the block counters stay
-    zero, and a configuration other than the plan runs in launches of 64."""
+    plan given as a configuration are bit-identical, the block counters end at
+    zero (130 and 192 rows: the last launch, of 2 and 64, counts its splits
+    there, in a workspace that the tile kernel's sums have passed through), and
+    a configuration other than the plan runs in launches of 64."""
     N, K = 2560, 4096
     say("forms", M)
     x, w = R.randn_bf16((M, K), 9900).to(device), R.randn_bf16((N, K), 9901, 0.02).to(device)
