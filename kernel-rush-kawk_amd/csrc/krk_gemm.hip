@@ -575,24 +575,30 @@ TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
     return best;
 }
 
-// Partial sums of the tile kernel's launches in a call of M > 64 rows whose
-// plan is c: at most what the static scratch of krk_gemm_bf16_noalloc holds,
-// so that every form of a call cuts K alike, and none where the plan keeps K
-// whole, whose calls bring no workspace.
+// The cut of a launch of `rows` rows on the tile kernel in a call whose plan is
+// c, and whether it takes the place of launches of 64 rows.  Its partial sums
+// take at most what the static scratch of krk_gemm_bf16_noalloc holds, so that
+// every form of a call cuts K alike, and none where the plan keeps K whole,
+// whose calls bring no workspace.  Where two splits of whole tiles do not fit
+// (97-128 rows of 4033-4096 plain or 2017-2048 SwiGLU channels) a long K goes
+// to launches of 64, which split it: 4096 x 7320, 128 rows 42.7 us against 44.2;
+// 4080 x 11600 59.0 against 66.2; but 4066 x 6112, 97 rows 36.7 against 33.2.
+// Over 1950 shapes of 65-128 rows no other loses more than 3%.
 constexpr size_t kTallPartMax = KRK_NOALLOC_SCRATCH_BYTES - KRK_NOALLOC_COUNTER_BYTES;
-inline TallPlan tall_cut(int rows, int N, int K, int epilogue, const krk_gemm_config& c) {
-    return tall_plan(rows, N, K, epilogue, c.splits > 1 ? kTallPartMax : 0);
+constexpr int kTallWholeMaxK = 6656;
+bool tall_cut(int rows, int N, int K, int epilogue, const krk_gemm_config& c, TallPlan* p) {
+    *p = tall_plan(rows, N, K, epilogue, c.splits > 1 ? kTallPartMax : 0);
+    return c.splits == 1 || p->splits > 1 || K <= kTallWholeMaxK;
 }
 size_t tall_part(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
     size_t most = 0;
-    const int last = M % krk::kTileMaxRows;  // of the launches of 128 rows
-    for (int rows : {M < krk::kTileMaxRows ? M : krk::kTileMaxRows, last}) {
-        if (rows <= kMaxRowsPerLaunch) continue;
-        const TallPlan p = tall_cut(rows, N, K, epilogue, c);
-        if (p.splits > 1) {
-            const size_t bytes = p.splits * krk::tile_part_bytes(p.mt, p.nt, p.nblk);
-            if (bytes > most) most = bytes;
-        }
+    // Rows of the launches a call of M rows may have on this kernel.
+    for (int rows : {M < krk::kTileMaxRows ? M : krk::kTileMaxRows, M % krk::kTileMaxRows,
+                     kMaxRowsPerLaunch + M % kMaxRowsPerLaunch}) {
+        TallPlan p;
+        if (rows <= kMaxRowsPerLaunch || !tall_cut(rows, N, K, epilogue, c, &p) || p.splits == 1) continue;
+        const size_t bytes = p.splits * krk::tile_part_bytes(p.mt, p.nt, p.nblk);
+        if (bytes > most) most = bytes;
     }
     return most;
 }
@@ -1563,7 +1569,9 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     const bool tall = !fused && tall_call(M, N, K, epilogue, c);
     int rows = 0;
     for (int m0 = 0; m0 < M; m0 += rows) {
-        const bool tile = tall && (M - m0 > kMaxRowsPerLaunch || M <= kMaxRowsPerLaunch);
+        TallPlan cut{};
+        const bool tile = tall && (M - m0 > kMaxRowsPerLaunch || M <= kMaxRowsPerLaunch) &&
+                          tall_cut(M - m0 < krk::kTileMaxRows ? M - m0 : krk::kTileMaxRows, N, K, epilogue, c, &cut);
         const int most = tile ? krk::kTileMaxRows : kMaxRowsPerLaunch;
         rows = M - m0 < most ? M - m0 : most;
         LaunchArgs a;
@@ -1581,7 +1589,7 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
         a.ctr = ctr;
         a.cb = g.cb;
         if (tile) {
-            rc = dispatch_tile(a, epilogue, tall_cut(rows, N, K, epilogue, c), st);
+            rc = dispatch_tile(a, epilogue, cut, st);
         } else if (fused) {
             // This chunk's rows of d and xout.
             krk::NormArgs nc = na;

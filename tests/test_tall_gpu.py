@@ -40,6 +40,24 @@ def test_gateup_rows_beyond_64(device, M, I, K):
     check_gateup(x, wgu, f"tall gateup M={M} I={I} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K,epi", [(128, 4096, 7320, NONE), (100, 4040, 9728, NONE), (200, 2 * 2040, 7168, SILU)])
+def test_long_k_beside_too_many_channels_to_split(device, M, N, K, epi):
+    """Two K splits of whole tiles do not fit the scratch of these calls, and
+    K is long: launches of 64 rows, which split it, are faster.  Their results
+    are those of 64-row calls bit for bit (up to the last launch of 200 rows,
+    whose 72 rows fit)."""
+    say("launches of 64", M, N, K, epi)
+    x, w = R.randn_bf16((M, K), 9260 + M).to(device), R.randn_bf16((N, K), 9360 + K, 0.02).to(device)
+    make = (lambda m: G.SkinnyGateUp(m, N // 2, K, device)) if epi == SILU else (lambda m: G.SkinnyMatmul(m, N, K, device))
+    assert G.plan(64, N, K, epi)["splits"] > 1
+    y = make(M)(x, w)
+    assert torch.equal(y[:64], make(64)(x[:64], w))
+    if M <= 128:
+        assert torch.equal(y[64:], make(64)(torch.cat([x[64:], x[:128 - M]]), w)[:M - 64])
+    ref = R.gateup_bf16(x.cpu(), w.cpu()) if epi == SILU else R.linear_bf16(x.cpu(), w.cpu())
+    assert_parity(y.cpu(), ref, "launches of 64")
+
+
 @pytest.mark.parametrize("M,N,K,epi", [
     (49, 16385, 72, NONE), (64, 20480, 520, NONE), (63, 18000, 2568, NONE),
     (49, 2 * 8193, 136, SILU), (64, 2 * 10240, 264, SILU), (60, 2 * 9001, 2632, SILU),
