@@ -156,10 +156,14 @@ typedef struct krk_gemm_config {
  * static shape -> kernel table that stands in for the reference's warm-up
  * pickers, engine/kernels/gemm.py:417-458, 461-498).  Returns KRK_OK or a
  * negative error for an invalid shape.  For more than 64 rows it describes the
- * launches of up to 64 rows; calls with it (or with no configuration) take
- * their larger launches on the tile kernel, whose own tiles follow from the
- * shape, and so do some shapes of 49 to 64 rows.  Any other configuration
- * runs in launches of up to 64 rows on its own kernel.
+ * launches of up to 64 rows, but for `splits` where that plan splits K: there
+ * it is the number of splits whose sums fill the workspace, which the larger
+ * launches use, and the launches of up to 64 rows split K as the 64-row plan
+ * does.  Calls with it (or with no configuration) take their larger launches
+ * on the tile kernel, whose own tiles follow from the shape (a few shapes
+ * with a long K run launches of 64 instead), and so do some shapes of 49 to 64
+ * rows.  Any other configuration runs in launches of up to 64 rows on its own
+ * kernel.
  */
 int krk_gemm_plan(int M, int N, int K, int epilogue, krk_gemm_config* out);
 

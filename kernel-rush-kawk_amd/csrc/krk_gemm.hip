@@ -254,6 +254,8 @@ inline int valu_depth(int MX, int R, int blocks) {
 }
 
 int stream_xs(int MT, int nst);
+int stream_max_depth(int MT, int nred);
+int stream_nred_for(int K, int splits);
 
 // Dynamic LDS a gfx950 workgroup may use: 160 KB less room for the kernels'
 // static __shared__ variables.
@@ -531,10 +533,6 @@ bool tile_rows_ok(int M, int N, int epilogue, const krk_gemm_config& c) {
     return per_cu > 4 * unit && per_cu <= krk::kTileMaxNT * unit;
 }
 
-void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
-    chunk_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue, c);
-}
-
 // How one launch of the tile kernel cuts `rows` (49..128) rows: tiles, output
 // channels per block and K splits, whose partial sums fit part_bytes.
 struct TallPlan {
@@ -575,32 +573,65 @@ TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
     return best;
 }
 
-// The cut of a launch of `rows` rows on the tile kernel in a call whose plan is
-// c, and whether it takes the place of launches of 64 rows.  Its partial sums
-// take at most what the static scratch of krk_gemm_bf16_noalloc holds, so that
-// every form of a call cuts K alike, and none where the plan keeps K whole,
-// whose calls bring no workspace.  Where two splits of whole tiles do not fit
-// (97-128 rows of 4033-4096 plain or 2017-2048 SwiGLU channels) a long K goes
-// to launches of 64, which split it: 4096 x 7320, 128 rows 42.7 us against 44.2;
-// 4080 x 11600 59.0 against 66.2; but 4066 x 6112, 97 rows 36.7 against 33.2.
-// Over 1950 shapes of 65-128 rows no other loses more than 3%.
+// Partial sums of a cut.
+inline size_t cut_bytes(const TallPlan& p) {
+    return p.splits > 1 ? p.splits * krk::tile_part_bytes(p.mt, p.nt, p.nblk) : 0;
+}
+
+// The cut of a launch of `rows` rows on the tile kernel in a call of M rows, and
+// whether it takes the place of launches of 64 rows.  split: the 64-row plan
+// splits K.  The partial sums take at most what the static scratch of
+// krk_gemm_bf16_noalloc holds, so that every form of a call cuts K alike, and
+// what the launches of 128 rows take in a smaller launch after them; none
+// where the 64-row plan keeps K whole, whose calls bring no workspace.  Where
+// two splits of whole tiles do not fit (97-128 rows of 4033-4096 plain or
+// 2017-2048 SwiGLU channels) a long K goes to launches of 64, which split it:
+// 4096 x 7320, 128 rows 42.7 us against 44.2; 4080 x 11600 59.0 against 66.2; but
+// 4066 x 6112, 97 rows 36.7 against 33.2.  Over 1950 shapes of 65-128 rows no
+// other loses more than 3%.
 constexpr size_t kTallPartMax = KRK_NOALLOC_SCRATCH_BYTES - KRK_NOALLOC_COUNTER_BYTES;
 constexpr int kTallWholeMaxK = 6656;
-bool tall_cut(int rows, int N, int K, int epilogue, const krk_gemm_config& c, TallPlan* p) {
-    *p = tall_plan(rows, N, K, epilogue, c.splits > 1 ? kTallPartMax : 0);
-    return c.splits == 1 || p->splits > 1 || K <= kTallWholeMaxK;
+bool tall_cut(int M, int rows, int N, int K, int epilogue, bool split, TallPlan* p) {
+    size_t most = split ? kTallPartMax : 0;
+    if (split && M > krk::kTileMaxRows && rows < krk::kTileMaxRows) {
+        const size_t first = cut_bytes(tall_plan(krk::kTileMaxRows, N, K, epilogue, kTallPartMax));
+        if (first) most = first;
+    }
+    *p = tall_plan(rows, N, K, epilogue, most);
+    return !split || p->splits > 1 || K <= kTallWholeMaxK;
 }
-size_t tall_part(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
+// The most partial sums of the launches a call of M > 64 rows may have there.
+size_t tall_part(int M, int N, int K, int epilogue, bool split) {
     size_t most = 0;
-    // Rows of the launches a call of M rows may have on this kernel.
     for (int rows : {M < krk::kTileMaxRows ? M : krk::kTileMaxRows, M % krk::kTileMaxRows,
                      kMaxRowsPerLaunch + M % kMaxRowsPerLaunch}) {
         TallPlan p;
-        if (rows <= kMaxRowsPerLaunch || !tall_cut(rows, N, K, epilogue, c, &p) || p.splits == 1) continue;
-        const size_t bytes = p.splits * krk::tile_part_bytes(p.mt, p.nt, p.nblk);
-        if (bytes > most) most = bytes;
+        if (rows <= kMaxRowsPerLaunch || !tall_cut(M, rows, N, K, epilogue, split, &p)) continue;
+        if (cut_bytes(p) > most) most = cut_bytes(p);
     }
     return most;
+}
+
+// The plan of launches of up to 64 rows.
+void launch_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
+    chunk_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue, c);
+}
+
+// The plan of a call.  For more than 64 rows, where the 64-row plan splits K,
+// it names the splits whose partial sums of 64 rows are the size of its
+// workspace, which has room for the tile kernel's; its launches of up to 64
+// rows split K as the 64-row plan does.
+void auto_config(int M, int N, int K, int epilogue, krk_gemm_config* c) {
+    launch_config(M, N, K, epilogue, c);
+    if (M <= kMaxRowsPerLaunch || c->splits == 1) return;
+    const size_t one = (size_t)kMaxRowsPerLaunch * N * sizeof(float);
+    const size_t need = tall_part(M, N, K, epilogue, true);
+    const bool stream = c->kernel == KRK_KERNEL_STREAM;
+    const int most = cdiv(K, stream ? krk::kStreamKC : 256) < 32 ? cdiv(K, stream ? krk::kStreamKC : 256) : 32;
+    int sp = c->splits;
+    while (sp < most && sp * one < need && (sp + 1) * one <= kTallPartMax) ++sp;
+    while (stream && sp > c->splits && c->unroll > stream_max_depth(c->m_tiles, stream_nred_for(K, sp))) --sp;
+    c->splits = sp;
 }
 
 // MFMA_LDS with x held in registers for the whole K (x_preload = 2): 512-k
@@ -621,14 +652,14 @@ int stream_xs(int MT, int nst) {
     return 0;
 }
 // Deepest ring that leaves room for one output-buffer block.
-inline int stream_max_depth(int MT, int nred) {
+int stream_max_depth(int MT, int nred) {
     int d = krk::kStreamMaxDepth;
     while (d > 2 && krk::stream_lds_bytes(MT, d, nred) + krk::stream_out_bytes(MT, false) > kLdsMax) --d;
     return d;
 }
 // Reduction areas of a stream launch: one when every split owns two or more
 // K stages.
-inline int stream_nred_for(int K, int splits) { return krk::stream_nred(cdiv(K, krk::kStreamKC) / splits); }
+int stream_nred_for(int K, int splits) { return krk::stream_nred(cdiv(K, krk::kStreamKC) / splits); }
 // Persistent grid: workgroups per split, at most one per CU, chosen so the
 // blocks divide as evenly as possible (a 1.25x overload costs more than
 // leaving CUs idle).
@@ -841,11 +872,17 @@ int complete_config(int M, int N, int K, int epilogue, const krk_gemm_config& a,
 // A caller's configuration with its zero fields filled from the plan, or
 // where that is none this build runs, from filler_config.
 int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in, krk_gemm_config* out) {
-    krk_gemm_config a;
-    auto_config(M, N, K, epilogue, &a);
-    if (!in) { *out = a; return KRK_OK; }
+    krk_gemm_config plan, a;
+    auto_config(M, N, K, epilogue, &plan);
+    if (!in) { *out = plan; return KRK_OK; }
+    launch_config(M, N, K, epilogue, &a);
     const int rc = complete_config(M, N, K, epilogue, a, in, out);
-    if (rc == KRK_OK) return rc;
+    if (rc == KRK_OK) {
+        // The plan in all but its splits, which the caller left open.
+        a.prologue = out->prologue;
+        if (!in->splits && !memcmp(out, &a, sizeof a)) out->splits = plan.splits;
+        return rc;
+    }
     krk_gemm_config f;
     filler_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue == KRK_EPILOGUE_SILU_MUL, &f);
     if (complete_config(M, N, K, epilogue, f, in, out) == KRK_OK) {
@@ -867,13 +904,14 @@ bool tall_call(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
 }
 
 // Workspace layout: [block counters, padded to 256 B][fp32 partials: splits x
-// Mc x N, or the tile kernel's where they are more].
+// Mc x N, or the tile kernel's where they are more (a multiple of 64 rows that
+// does not fit the static scratch)].
 size_t workspace_for(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
     if (c.splits <= 1) return 0;
     const Geometry g = geometry(M, N, epilogue, c);
     size_t part = (size_t)c.splits * (size_t)g.Mc * (size_t)N * sizeof(float);
     if (M > kMaxRowsPerLaunch && tall_call(M, N, K, epilogue, c)) {
-        const size_t tall = tall_part(M, N, K, epilogue, c);
+        const size_t tall = tall_part(M, N, K, epilogue, true);
         if (tall > part) part = tall;
     }
     return align_up((size_t)g.nblocks * sizeof(uint32_t), 256) + part;
@@ -1567,11 +1605,17 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     // launches of up to 128 rows on the tile kernel while more than 64 are left.
     // 49 to 64 rows: one launch of it where tile_rows_ok says so.
     const bool tall = !fused && tall_call(M, N, K, epilogue, c);
+    if (tall) {  // the plan's launches of up to 64 rows
+        krk_gemm_config l;
+        launch_config(M, N, K, epilogue, &l);
+        c.splits = l.splits;
+    }
     int rows = 0;
     for (int m0 = 0; m0 < M; m0 += rows) {
         TallPlan cut{};
         const bool tile = tall && (M - m0 > kMaxRowsPerLaunch || M <= kMaxRowsPerLaunch) &&
-                          tall_cut(M - m0 < krk::kTileMaxRows ? M - m0 : krk::kTileMaxRows, N, K, epilogue, c, &cut);
+                          tall_cut(M, M - m0 < krk::kTileMaxRows ? M - m0 : krk::kTileMaxRows, N, K, epilogue,
+                                   c.splits > 1, &cut);
         const int most = tile ? krk::kTileMaxRows : kMaxRowsPerLaunch;
         rows = M - m0 < most ? M - m0 : most;
         LaunchArgs a;
@@ -1687,7 +1731,7 @@ constexpr int kStreamSelDepth = 5;
 
 int select_plan_for(int M, int N, int K, int k, const krk_gemm_config* cfg, SelectPlan* out) {
     const int Mc = M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch;
-    int rc = resolve_config(M, N, K, KRK_EPILOGUE_NONE, cfg, &out->c);
+    int rc = resolve_config(Mc, N, K, KRK_EPILOGUE_NONE, cfg, &out->c);
     if (rc) return rc;
     out->fused = select_fusable(out->c, Mc, K, k);
     if (!cfg && out->fused && out->c.kernel == KRK_KERNEL_STREAM && out->c.unroll > kStreamSelDepth)

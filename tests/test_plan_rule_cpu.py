@@ -62,21 +62,30 @@ def test_partial_configurations_are_completed(M, N, K, epi, cfg):
     assert again.as_dict() == out
 
 
-def test_plans_beyond_64_rows_are_the_64_row_plans():
-    """A call of more than 64 rows runs its last launch, of up to 64, on the
-    64-row plan, K splits included; what the larger launches need on top only
-    shows in the workspace, which stays within the static scratch."""
+def test_splits_beyond_64_rows():
+    """A plan for more than 64 rows is the 64-row plan but for its splits, which
+    size the workspace for the tile kernel's sums; what runs in launches of 64
+    rows (a selecting call, a configuration with other fields than the plan's)
+    splits K as the 64-row plan does."""
     lib = _lib.load()
-    shapes = [(130, 2560, 4096), (192, 2560, 9728), (66, 1938, 7896)] + list(_shapes(17, 2000))
+    shapes = [(130, 2560, 4096), (192, 2560, 9728), (66, 1938, 7896), (112, 536, 10008)] + list(_shapes(17, 2000))
     for M, N, K in shapes:
         M = 65 + M % 192
+        plan, base, got = GemmConfig(), GemmConfig(), GemmConfig()
         for epi in (NONE, SILU):
-            plan, base = GemmConfig(), GemmConfig()
             assert lib.krk_gemm_plan(M, N, K, epi, ctypes.byref(plan)) == 0
             assert lib.krk_gemm_plan(64, N, K, epi, ctypes.byref(base)) == 0
-            assert plan.as_dict() == base.as_dict(), (M, N, K, epi)
+            p, b = plan.as_dict(), base.as_dict()
+            assert dict(p, splits=0) == dict(b, splits=0) and p["splits"] >= b["splits"], (M, N, K, epi)
             need, need64 = lib.krk_gemm_workspace_bytes(M, N, K, epi), lib.krk_gemm_workspace_bytes(64, N, K, epi)
             assert need64 <= need <= max(need64, 4 << 20), (M, N, K, epi)
+            for cfg, splits in (({}, p["splits"]), ({"kernel": p["kernel"]}, p["splits"]), (p, p["splits"])):
+                given = GemmConfig.from_dict(cfg)
+                assert lib.krk_gemm_resolve(M, N, K, epi, ctypes.byref(given), ctypes.byref(got)) == 0
+                assert got.as_dict() == dict(p, splits=splits), (M, N, K, epi, cfg)
+            other = GemmConfig.from_dict(dict(p, unroll=5 - p["unroll"] if p["kernel"] == _lib.KERNEL_MFMA_LDS else 2, splits=0))
+            if lib.krk_gemm_resolve(M, N, K, epi, ctypes.byref(other), ctypes.byref(got)) == 0 and got.unroll != plan.unroll:
+                assert got.splits == b["splits"], (M, N, K, epi, got.as_dict())
         if N >= 8:
             assert lib.krk_gemm_select_plan(M, N, K, 8, ctypes.byref(plan)) == 0
             assert lib.krk_gemm_select_plan(64, N, K, 8, ctypes.byref(base)) == 0
