@@ -363,6 +363,50 @@ void lds_rule(int mt, int nt, int unroll, int kc, int channels, int splits, int 
     r->x_preload = x_preload;
 }
 
+// Rows and channels for which the tile kernel is faster than an LDS-staged plan
+// with K whole (MI355X, graph replay over distinct weights, us): 49 rows and
+// more, 65-80 plain or 33-40 SwiGLU channels per CU.  Five tiles hold them in
+// one round of blocks, the plan's four take two (16400 x 6144, M = 64: 60.8 ->
+// 49.0; x 520: 15.9 -> 11.0; 10000 SwiGLU channels, K = 3072: 37.4 -> 31.2).  No
+// split, so no workspace.  Not taken here, though the tile kernel measured
+// faster: K up to ~1500 beside fewer channels (12288 x 1024, M = 64: 1.17x;
+// 18992 x 1536 in place of the stream plan: 1.04-1.12x) and split plans of a
+// long K (3072 x 8192: 1.17x, its sums do not fit the plan's workspace); at
+// longer K neither wins (14000 x 6144: 41.1, 42.9 here; 8192 SwiGLU channels,
+// K = 2560: 22.0, 22.6).  At 48 rows and fewer the plan has three x tiles and
+// wins or ties more often.
+constexpr int kTileMinRows = 49;
+bool tile_width_ok(int Mc, int Nout, bool silu) {
+    const int unit = silu ? 8 : 16;
+    const int per_cu = cdiv(Nout, kCuCount);
+    return Mc >= kTileMinRows && per_cu > 4 * unit && per_cu <= krk::kTileMaxNT * unit;
+}
+
+// 33-64 rows of a long weight stream whose K is below 1024: the stream kernel
+// instead of LDS-staged blocks.  It pays for whole 512-k stages, the other for
+// 256-k ones, and its stores are wide only where the rows of y (ldy = Nout)
+// stay 16-byte aligned.  Times of both (us, stream / LDS-staged):
+//   * K <= 256: never (48697 SwiGLU channels, K = 256, M = 62: 48.8 / 34.8;
+//     over 220 such shapes the stream kernel took 0.97-1.67x the time);
+//   * aligned rows, K > 256: always (34784 SwiGLU channels, K = 352, M = 41:
+//     24.7 / 32.0; 137168 x 384, M = 47: 45.1 / 57.4; 119680 x 456, M = 39: 40.1
+//     / 53.9);
+//   * other rows: past K = 768 (53938 channels, K = 968, M = 43: 60.5 / 74.4),
+//     and with three x tiles where K does not leave most of a 512-k stage
+//     empty (26268 channels, K = 488, M = 36: 24.4 / 28.7; 33174, K = 760, M =
+//     35: 37.1 / 41.7), as it does elsewhere (14497 channels, K = 576, M = 52:
+//     22.5 / 17.8);
+//   * where the tile kernel takes the LDS-staged plan's place (tile_rows_ok):
+//     past K = 768, other rows just below 1024 (10016 channels, K = 1000, M =
+//     49: 16.1 / 17.9; 9943, K = 1016: 18.1 / 19.2; but 8200, K = 640, M = 60:
+//     14.6 / 12.7; 9047, K = 784: 17.7 / 16.6).
+bool short_stream(int Mc, int Nout, int K, bool silu) {
+    if (Mc <= 32 || K <= 256) return false;
+    const bool aligned = Nout % 8 == 0;
+    if (tile_width_ok(Mc, Nout, silu)) return K > (aligned ? 768 : 992);
+    return aligned || K > 768 || (Mc <= 48 && ((K > 352 && K <= 512) || K > 704));
+}
+
 void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
     const int mt = cdiv(Mc, 16);
     const int KST = cdiv(K, 512);
@@ -382,8 +426,10 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
         // 33 rows and more, few channels go to the stream kernel's blocks of
         // 8 (268 channels, K = 1608, M = 37: 8.6 against 9.2), and so do more
         // than one round holds while x fits its registers with K whole (12105
-        // channels, K = 1432, M = 39: 19.9 against 23.5).
-        if ((Mc > 32 && Nout <= 1200) || (Nout > 32 * kCuCount && K >= 1024 && stream_xs(mt, KST))) {
+        // channels, K = 1432, M = 39: 19.9 against 23.5), below K = 1024 as
+        // short_stream says.
+        if ((Mc > 32 && Nout <= 1200) ||
+            (Nout > 32 * kCuCount && (K >= 1024 ? stream_xs(mt, KST) > 0 : short_stream(Mc, Nout, K, true)))) {
             c->kernel = KRK_KERNEL_STREAM;
             c->m_tiles = mt;
             c->n_tiles = 1;
@@ -435,7 +481,8 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
         return;
     }
     if (Mc <= 4 || (Mc <= kValuMaxRows && per_cu > kSliceMaxChannels)) return valu_rule(Mc, N, K, false, c);
-    if (N >= 64 * kCuCount && K >= 1024 && stream_xs(mt, KST)) {
+    if ((N >= 64 * kCuCount && K >= 1024 && stream_xs(mt, KST)) ||
+        (N >= 256 * kCuCount && K < 1024 && short_stream(Mc, N, K, false))) {
         // A long weight stream and x that fits the registers with K whole
         // (37984 x 2560, M = 10 / 32 / 64: 34.4 / 39.0 / 43.8 against 45.2 /
         // 49.0 / 61.9 on 32-channel LDS-staged blocks).
@@ -515,22 +562,11 @@ void chunk_config(int Mc, int N, int K, int epilogue, krk_gemm_config* c) {
     rule_config(Mc, N, K, silu, c);
 }
 
-// 49 to 64 rows that run on the tile kernel in place of the LDS-staged plan
-// (MI355X, graph replay over distinct weights, us): 65-80 plain or 33-40
-// SwiGLU channels per CU with K whole.  Five tiles hold them in one round of
-// blocks, the plan's four take two (16400 x 6144, M = 64: 60.8 -> 49.0;
-// x 520: 15.9 -> 11.0; 10000 SwiGLU channels, K = 3072: 37.4 -> 31.2).  At
-// four tiles and fewer both run one round and neither wins (14000 x 6144:
-// 41.1, 42.9 here; 8192 SwiGLU channels, K = 2560: 22.0, 22.6).  No split, so
-// no workspace.
-// At 48 rows and fewer the plan has three x tiles and wins or ties more often.
-constexpr int kTileMinRows = 49;
+// 49 to 64 rows that run on the tile kernel in place of the LDS-staged plan.
 bool tile_rows_ok(int M, int N, int epilogue, const krk_gemm_config& c) {
-    if (M < kTileMinRows || M > kMaxRowsPerLaunch || c.kernel != KRK_KERNEL_MFMA_LDS || c.splits > 1) return false;
     const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
-    const int unit = silu ? 8 : 16;
-    const int per_cu = cdiv(silu ? N / 2 : N, kCuCount);
-    return per_cu > 4 * unit && per_cu <= krk::kTileMaxNT * unit;
+    return M <= kMaxRowsPerLaunch && c.kernel == KRK_KERNEL_MFMA_LDS && c.splits == 1 &&
+           tile_width_ok(M, silu ? N / 2 : N, silu);
 }
 
 // How one launch of the tile kernel cuts `rows` (49..128) rows: tiles, output

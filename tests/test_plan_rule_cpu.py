@@ -62,6 +62,23 @@ def test_partial_configurations_are_completed(M, N, K, epi, cfg):
     assert again.as_dict() == out
 
 
+@pytest.mark.parametrize("M,N,K,epi,stream", [
+    (44, 153720, 792, NONE, True), (51, 153320, 384, NONE, True), (49, 115344, 568, NONE, True),   # aligned rows of y
+    (41, 2 * 34784, 352, SILU, True), (37, 2 * 52032, 816, SILU, True), (64, 2 * 31272, 760, SILU, True),
+    (43, 2 * 53938, 968, SILU, True), (36, 2 * 26268, 488, SILU, True), (36, 2 * 26268, 512, SILU, True),   # others
+    (35, 2 * 33174, 760, SILU, True), (45, 2 * 41095, 376, SILU, True), (49, 2 * 9943, 1016, SILU, True),
+    (62, 2 * 48697, 256, SILU, False), (52, 2 * 14497, 576, SILU, False), (62, 2 * 26268, 488, SILU, False),
+    (44, 144278, 200, NONE, False), (44, 65528, 792, NONE, False), (32, 153720, 792, NONE, False),
+    (64, 2 * 9000, 1000, SILU, True), (49, 2 * 10016, 776, SILU, True),   # where the tile kernel is the other choice
+    (60, 2 * 8200, 640, SILU, False), (49, 2 * 9047, 784, SILU, False), (48, 2 * 9000, 640, SILU, True),
+])
+def test_wide_shapes_of_a_short_k(M, N, K, epi, stream):
+    """33-64 rows below K = 1024: the stream kernel where it measured faster."""
+    plan = GemmConfig()
+    assert _lib.load().krk_gemm_plan(M, N, K, epi, ctypes.byref(plan)) == 0
+    assert plan.kernel == (_lib.KERNEL_STREAM if stream else _lib.KERNEL_MFMA_LDS), plan.as_dict()
+
+
 def test_splits_beyond_64_rows():
     """A plan for more than 64 rows is the 64-row plan but for its splits, which
     size the workspace for the tile kernel's sums; what runs in launches of 64

@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
     (5, 255, 72), (12, 4096, 1416), (13, 4104, 1416), (16, 8192, 520), (32, 8200, 520), (8, 8300, 2056),
     (9, 600, 6672), (17, 1800, 4104), (24, 3300, 4104), (32, 500, 5128),                   # LDS-staged, split
     (33, 1023, 1536), (33, 1024, 3072), (64, 2047, 2048), (48, 2048, 3080), (40, 5000, 1544), (64, 9000, 1528),
-    (16, 16390, 1024), (33, 16400, 1000),                                                  # stream
+    (16, 16390, 1024), (33, 16400, 1000), (33, 65536, 264), (49, 65544, 1016),              # stream
 ])
 def test_rule_plans(device, M, N, K):
     x, w = R.randn_bf16((M, K), 8100 + M + N), R.randn_bf16((N, K), 8200 + K, 0.02)
@@ -30,6 +30,7 @@ def test_rule_plans(device, M, N, K):
     (1, 1025, 2824), (2, 300, 5640), (4, 2100, 1544), (6, 310, 4104), (8, 1201, 2560),     # VALU
     (9, 4097, 520), (16, 300, 2560), (17, 2050, 4096), (32, 1300, 3600), (32, 500, 1800),  # LDS-staged
     (33, 1200, 1000), (33, 1201, 1000), (64, 4500, 1032), (40, 8300, 1032),                # stream / LDS-staged
+    (36, 8200, 264), (48, 8195, 512), (64, 8200, 776), (50, 10248, 264), (64, 8199, 1016),
 ])
 def test_rule_gateup_plans(device, M, I, K):
     x, w = R.randn_bf16((M, K), 8300 + M + I), R.randn_bf16((2 * I, K), 8400 + K, 0.02)
