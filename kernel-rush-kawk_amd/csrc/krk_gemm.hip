@@ -1765,11 +1765,30 @@ struct SelectPlan {
 // 122 against 131 µs for top-8 with the 7 the plain plan uses).
 constexpr int kStreamSelDepth = 5;
 
+// Argmax of few channels at 33 rows and more: the plan's blocks of 8 or 16
+// channels on one weight tile have no selecting variant; 16 channels on two
+// (half of the second padding) select in the epilogue, and save the logits'
+// round trip (MI355X, graph replay, us: 1720 x 480, M = 33: 11.2 -> 7.9; 4076 x
+// 416, M = 40: 11.6 -> 8.3; 1904 x 1904, M = 48: 14.6 -> 12.6; 2214 x 2520, M = 56:
+// 17.7 -> 14.6; 137 shapes: 1.06-1.49x).  Not for plans on the stream
+// kernel without a selecting variant: the fused LDS-staged one is 1.0-1.4x
+// slower there (32618 x 1880, M = 50: 51.5 against 38.9).
 int select_plan_for(int M, int N, int K, int k, const krk_gemm_config* cfg, SelectPlan* out) {
     const int Mc = M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch;
     int rc = resolve_config(Mc, N, K, KRK_EPILOGUE_NONE, cfg, &out->c);
     if (rc) return rc;
     out->fused = select_fusable(out->c, Mc, K, k);
+    if (!cfg && !out->fused && Mc > 32 && out->c.kernel == KRK_KERNEL_MFMA_LDS && out->c.n_tiles == 1 &&
+        out->c.k_chunk == 256) {
+        krk_gemm_config wide = out->c;
+        wide.n_tiles = 2;
+        wide.channels = 16;
+        wide.unroll = 2;
+        if (select_fusable(wide, Mc, K, k)) {
+            out->c = wide;
+            out->fused = true;
+        }
+    }
     if (!cfg && out->fused && out->c.kernel == KRK_KERNEL_STREAM && out->c.unroll > kStreamSelDepth)
         out->c.unroll = kStreamSelDepth;
     return KRK_OK;

@@ -79,6 +79,16 @@ def test_wide_shapes_of_a_short_k(M, N, K, epi, stream):
     assert plan.kernel == (_lib.KERNEL_STREAM if stream else _lib.KERNEL_MFMA_LDS), plan.as_dict()
 
 
+@pytest.mark.parametrize("M,N,K", [(34, 1654, 752), (33, 1024, 64), (48, 2048, 1536), (64, 4096, 3072), (100, 3126, 1344)])
+def test_argmax_of_few_channels_is_fused(M, N, K):
+    lib, plan = _lib.load(), GemmConfig()
+    assert lib.krk_gemm_select_fused(M, N, K, 1, None) == 1
+    assert lib.krk_gemm_select_plan(M, N, K, 1, ctypes.byref(plan)) == 0
+    assert lib.krk_gemm_select_fused(M, N, K, 1, ctypes.byref(plan)) == 1
+    if N >= 8:
+        assert lib.krk_gemm_select_fused(M, N, K, 8, None) == 0
+
+
 def test_splits_beyond_64_rows():
     """A plan for more than 64 rows is the 64-row plan but for its splits, which
     size the workspace for the tile kernel's sums; what runs in launches of 64

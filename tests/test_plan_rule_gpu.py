@@ -8,7 +8,7 @@ import pytest
 
 from kernels import gemm as G
 from oracle import gemm_ref as R
-from test_gemm_gpu import check_gateup, check_linear
+from test_gemm_gpu import _check_selection, assert_parity, check_gateup, check_linear, krk_select, say
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,20 @@ def test_rule_plans(device, M, N, K):
 def test_rule_gateup_plans(device, M, I, K):
     x, w = R.randn_bf16((M, K), 8300 + M + I), R.randn_bf16((2 * I, K), 8400 + K, 0.02)
     check_gateup(x, w, f"rule {G.plan(M, 2 * I, K, 1)}")
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 1024, 64), (40, 2047, 520), (64, 4095, 1536), (100, 1554, 3072), (49, 3009, 776)])
+def test_fused_argmax_of_few_channels(device, M, N, K):
+    """Argmax in the epilogue on half-padded weight tiles: the oracle's choice
+    among the call's own logits, with equal maxima in one row and NaN in another,
+    and the same without the logits."""
+    x, w = R.randn_bf16((M, K), 8500 + M), R.randn_bf16((N, K), 8600 + N, 0.02)
+    w[N - 1], w[17] = w[5], w[5]      # equal logits in every row
+    x[M - 1, K - 1] = float("nan")
+    assert G.select_fused(M, N, K, 1)
+    say("fused argmax", M, N, K)
+    idx, vals, logits = krk_select(x, w, 1)
+    _check_selection(idx, vals, logits, 1, f"argmax M={M} N={N} K={K}")
+    assert_parity(logits[:M - 1], R.linear_bf16(x[:M - 1], w), "logits")
+    again, _, _ = krk_select(x, w, 1, logits=False)
+    assert again.tolist() == idx.tolist()
