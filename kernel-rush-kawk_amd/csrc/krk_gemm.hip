@@ -289,6 +289,25 @@ inline int even_channels(int Nout, int most) {
     return round8(cdiv(Nout, kCuCount * rounds));
 }
 
+// A VALU launch of few blocks (quads: of 4 waves) that would each walk a long K
+// (nb 512-blocks): K is split until about 600 run (307 SwiGLU channels, K =
+// 9600, M = 6: 9.6 with 8 splits, 14.6 whole; 24, K = 3504, M = 8: 5.8 / 7.8).  At
+// M = 1 a block that holds its rows in flight walks K fast: splits pay past K =
+// 11264 (SwiGLU; 300 channels, K = 15752: 9.0 / 12.5) or 15360 (plain; 300 x 15880:
+// 7.7 / 8.9) for 36-191 blocks, where up to 16 of them fill the CUs, and for a
+// handful of blocks (24 SwiGLU channels, K = 11768: 7.3 / 9.7); between them the
+// fix-up of 20-32 splits costs more than it gives.
+bool valu_starved(int Mc, int quads, int nb, bool silu) {
+    if (Mc == 1) {
+        if (quads <= 3 || (silu && quads <= 10)) return nb >= (!silu ? 22 : quads <= 6 ? 11 : 18);
+        return quads >= 36 && quads < 192 && nb >= (silu ? 23 : 31);
+    }
+    if (Mc == 2) return quads < 192 && nb >= 10;
+    if (Mc >= 5 && quads <= 16 && nb >= 6) return true;
+    if (nb >= 20) return quads < 320;  // 1195 SwiGLU channels, K = 14184, M = 3: 20.0 / 23.1
+    return quads < (Mc >= 5 && nb >= 13 ? 224 : 192) && nb >= (Mc <= 4 ? 8 : 7);
+}
+
 // VALU: a block of `waves` waves, one or two W rows each.
 //   * One row per wave: plain, M = 1 past 2560 channels (18280 x 3000: 19.0
 //     against 20.9 with two) and below 2048; else two (3072 x 2560, M = 2:
@@ -298,26 +317,37 @@ inline int even_channels(int Nout, int most) {
 //     M = 2: 6.44 with 5 waves, 6.87 with 4).  With x in LDS (M >= 3) the
 //     waves of a block share it: eight, plain (2560 x 2048, M = 4: 4.6
 //     against 4.8) unless a short K ends in part of a block (9518 x 2240, M =
-//     3: 10.2 with 4 waves of one row, 10.7 with 8 of two), and SwiGLU where x
-//     leaves a CU fewer than three blocks
-//     (12000 channels, K = 4096, M = 6: 33.5 with 8, 41.6 with 4).
-//   * K is split only where a few blocks would each walk a long K (307 SwiGLU
-//     channels, K = 9600, M = 6: 9.6 with 8 splits, 14.6 whole), and where x
-//     would leave a CU one or two blocks over 16 or more blocks of k.
-//   * Depth: blocks that fit one round hold all of a row in flight; with more
+//     3: 10.2 with 4 waves of one row, 10.7 with 8 of two; 4432 x 3160: 9.0,
+//     10.4) or five rows and more have one or three blocks of k (65536 x 512, M =
+//     6: 21.3 with 4, 24.7 with 8; x 1536: 36.5, 39.3; but x 1024, M = 8: 27.1,
+//     25.9), and SwiGLU where x leaves a CU fewer than three blocks (12000
+//     channels, K = 4096, M = 6: 33.5 with 8, 41.6 with 4).
+//   * K is split where valu_starved says so, and where x would leave a CU one
+//     or two blocks over 16 or more blocks of k.
+//   * Depth: blocks that fit one round hold all of a row in flight, and past 19
+//     blocks of k (10 with two rows of each x) the depth of 7 and 10 whose last
+//     pass is fuller (1002 x 11624, M = 1: 9.3 with 19, 8.3 with 7).  With more
 //     rounds other workgroups cover the latency and a depth past 7 only costs
-//     occupancy (6810 x 7120, M = 1: 16.8 with 2 in flight, 23.2 with 19;
-//     12288 x 4096: 15.8 with 4, 17.0 with 8).
+//     occupancy (6810 x 7120, M = 1: 16.8 with 2 in flight, 23.2 with 19; 12288 x
+//     4096: 15.8 with 4, 17.0 with 8) unless it saves the masked blocks of a
+//     last pass.  Over 4-24 blocks of k, M = 1-8, N = 6810-20000, depths 2-10: up
+//     to 5 blocks and 7 are best in one pass (2 takes up to 1.18x, 4 at 5 blocks
+//     1.22x), multiples of 4 at 4 (1.00-1.16x of the best; 8 ties 4 at 8 blocks,
+//     but takes 1.1x at M = 8), the rest at 2 or 3 (1.00-1.14x); at M = 1 one pass
+//     of 7 for 6 blocks and of 10 for 9 and 10 (1.00-1.10x, 2 takes up to 1.19x),
+//     and of 8 for 8 where the last is partial (4 takes 1.02-1.07x).
+//     Past 12 blocks, SwiGLU at M = 1 with a partial last block: 5 or 7 (8912
+//     channels, K = 8880: 62.0 -> 56.2 us).
 void valu_rule(int Mc, int N, int K, bool silu, krk_gemm_config* r) {
     const int Nout = silu ? N / 2 : N;
     const int nb = cdiv(K, krk::kValuBlock);
     r->kernel = KRK_KERNEL_VALU;
     r->m_tiles = valu_mx(Mc);
-    r->n_tiles = silu || (N > 8 * kCuCount && (Mc > 1 || N <= 10 * kCuCount || (N <= 16 * kCuCount && nb > 8))) ? 2 : 1;
+    r->n_tiles = silu || Mc > 4 || (N > 8 * kCuCount && (Mc > 1 || N <= 10 * kCuCount || (N <= 16 * kCuCount && nb > 8))) ? 2 : 1;
     const int per_wave = silu ? 1 : r->n_tiles;
     r->splits = 1;
     const int quads = cdiv(Nout, 4 * per_wave);  // blocks of 4 waves
-    const bool starved = Mc >= 2 && quads < 192 && nb >= (Mc == 2 ? 10 : 8);
+    const bool starved = valu_starved(Mc, quads, nb, silu);
     const size_t fit = Mc >= 3 && nb >= 16 ? kLdsBudget : kLdsMax;
     while (r->splits < nb && r->splits < 32 &&
            ((starved && quads * r->splits < 600) || krk::valu_lds_bytes(r->m_tiles, cdiv(nb, r->splits)) > fit))
@@ -332,8 +362,10 @@ void valu_rule(int Mc, int N, int K, bool silu, krk_gemm_config* r) {
     const int one_round = cdiv(Nout, kCuCount * per_wave);  // waves of a single round's blocks
     const bool single = one_round <= krk::kValuMaxWaves;
     const bool whole = K % krk::kValuBlock == 0;
-    if (Mc >= 3 && !silu && !single && !whole && nb <= 5) {
+    if (Mc >= 3 && !silu && !single && !whole && (nb <= 5 || (nb == 7 && Mc <= 4 && N <= 64 * kCuCount))) {
         r->n_tiles = Mc <= 4 ? 1 : 2;
+        r->waves = 4;
+    } else if (Mc > 4 && !silu && whole && (nb == 1 || nb == 3)) {
         r->waves = 4;
     } else if (Mc >= 3 && (!silu || lds > kLdsMax / 3)) {
         r->waves = krk::kValuMaxWaves;
@@ -345,10 +377,14 @@ void valu_rule(int Mc, int N, int K, bool silu, krk_gemm_config* r) {
             for (int wv : {5, 6})
                 if (round_fill(cdiv(Nout, wv * per_wave)) > round_fill(cdiv(Nout, r->waves * per_wave)) + 0.02) r->waves = wv;
     }
-    if (per <= 5 || per == 7 || (single && Mc <= 2) || (Mc == 1 && (per == 6 || per == 9 || per == 10 || (per == 8 && !whole))))
+    const bool covers = per <= 5 || per == 7 || (Mc == 1 && (per == 6 || per == 9 || per == 10 || (per == 8 && !whole)));
+    if (covers || (single && Mc <= 2))
         r->unroll = valu_depth(r->m_tiles, r->n_tiles, per);
+    else if (silu && Mc == 1 && !whole && per > 12 && Nout > 16 * kCuCount)
+        r->unroll = cdiv(per, 7) * 7 < cdiv(per, 5) * 5 ? 7 : 5;
     else
         r->unroll = per % 4 == 0 ? 4 : 2;
+    if (r->unroll < per && single && Mc <= 2) r->unroll = cdiv(per, 7) * 7 < cdiv(per, 10) * 10 ? 7 : 10;
 }
 
 void lds_rule(int mt, int nt, int unroll, int kc, int channels, int splits, int x_preload, krk_gemm_config* r) {
@@ -460,9 +496,16 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
     // or K is long for 9-32 rows (400 x 9728, M = 32: 8.6 with 8 LDS-staged
     // splits, over 10.8 here; 1984 x 9880, M = 15: 13.6 against 15.3).
     const int per_cu = cdiv(N, kCuCount);
-    const bool few_rows = Mc >= 3 && Mc <= 4 && N <= 16 * kCuCount &&
+    // A handful of blocks that each walk a long K, and few channels past K =
+    // 11264 (3-4 rows) or 13824, go to the VALU kernel, which splits it (26 x
+    // 13640, M = 5: 7.3 against 9.3; 16 x 14704, M = 4: 7.2 / 9.1; 210 x 14600, M =
+    // 3: 8.7 / 9.9; 400 x 15528, M = 7: 10.0 / 11.4; 44 x 9688, M = 3 stays: 1.08x).
+    const bool narrow = Mc <= 4 ? (K > 7000 && N * 320 < K) || (K > 11264 && N > 128 && N <= 768)
+                                : Mc <= kValuMaxRows && ((K > 7000 && N * 192 < K) ||
+                                                         (K > 13824 && N >= 256 && N <= 768));
+    const bool few_rows = Mc >= 3 && Mc <= 4 && N <= 16 * kCuCount && !narrow &&
                           (K > 3072 || (K > 1024 && K % krk::kValuBlock != 0));
-    const bool sliced = Mc >= 5 && Mc <= 32 && per_cu <= kSliceMaxChannels && !(per_cu > 16 && K > 4096) &&
+    const bool sliced = Mc >= 5 && Mc <= 32 && per_cu <= kSliceMaxChannels && !(per_cu > 16 && K > 4096) && !narrow &&
                         !(Mc > 8 && K > 6656) &&
                         !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 8 || per_cu > 12))));
     const bool wide_sliced = Mc >= 5 && Mc <= 8 && per_cu > kSliceMaxChannels && K >= 2048 && K <= 8192;
@@ -480,7 +523,7 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
         c->m_tiles = v.MT;
         return;
     }
-    if (Mc <= 4 || (Mc <= kValuMaxRows && per_cu > kSliceMaxChannels)) return valu_rule(Mc, N, K, false, c);
+    if (Mc <= 4 || narrow || (Mc <= kValuMaxRows && per_cu > kSliceMaxChannels)) return valu_rule(Mc, N, K, false, c);
     if ((N >= 64 * kCuCount && K >= 1024 && stream_xs(mt, KST)) ||
         (N >= 256 * kCuCount && K < 1024 && short_stream(Mc, N, K, false))) {
         // A long weight stream and x that fits the registers with K whole

@@ -79,6 +79,41 @@ def test_wide_shapes_of_a_short_k(M, N, K, epi, stream):
     assert plan.kernel == (_lib.KERNEL_STREAM if stream else _lib.KERNEL_MFMA_LDS), plan.as_dict()
 
 
+@pytest.mark.parametrize("M,N,K,epi,splits", [
+    (1, 600, 15752, SILU, 8), (1, 10, 9736, SILU, 20), (8, 48, 3504, SILU, 7), (7, 20, 2632, SILU, 6),
+    (3, 2390, 14184, SILU, 3), (1, 300, 15880, NONE, 8), (5, 26, 13640, NONE, 27), (8, 36, 7888, NONE, 16),
+    (3, 210, 14600, NONE, 12), (4, 16, 14704, NONE, 29),
+    (1, 320, 12296, SILU, 15), (7, 400, 15528, NONE, 12), (3, 1550, 12656, SILU, 4),
+    (1, 160, 12296, SILU, 1), (1, 300, 12296, NONE, 1), (3, 44, 9688, NONE, 1),
+])
+def test_few_channels_of_a_long_k(M, N, K, epi, splits):
+    """Up to 8 rows: K is split where a few blocks would each walk all of it."""
+    plan = GemmConfig()
+    assert _lib.load().krk_gemm_plan(M, N, K, epi, ctypes.byref(plan)) == 0
+    assert plan.splits == splits, plan.as_dict()
+    assert splits == 1 or plan.kernel == _lib.KERNEL_VALU
+
+
+@pytest.mark.parametrize("M,N,K,epi,depth", [
+    (1, 1002, 11624, NONE, 7), (1, 1002, 10240, NONE, 10), (1, 1002, 9728, NONE, 19), (2, 1600, 10752, NONE, 7),
+    (1, 1600, 10752, SILU, 7), (1, 1600, 10240, SILU, 10), (1, 2 * 8912, 8880, SILU, 5), (1, 2 * 8912, 10300 // 8 * 8, SILU, 7),
+])
+def test_depth_past_one_pass(M, N, K, epi, depth):
+    plan = GemmConfig()
+    assert _lib.load().krk_gemm_plan(M, N, K, epi, ctypes.byref(plan)) == 0
+    assert plan.kernel == _lib.KERNEL_VALU and plan.unroll == depth, plan.as_dict()
+
+
+@pytest.mark.parametrize("M,N,K,waves,rows", [
+    (6, 65536, 512, 4, 2), (8, 10240, 1536, 4, 2), (8, 65536, 1024, 8, 2), (4, 65536, 512, 8, 2),
+    (3, 4432, 3160, 4, 1), (3, 16390, 3160, 8, 2), (3, 8982, 3584, 8, 2),
+])
+def test_waves_of_many_channels(M, N, K, waves, rows):
+    plan = GemmConfig()
+    assert _lib.load().krk_gemm_plan(M, N, K, NONE, ctypes.byref(plan)) == 0
+    assert (plan.kernel, plan.waves, plan.n_tiles) == (_lib.KERNEL_VALU, waves, rows), plan.as_dict()
+
+
 @pytest.mark.parametrize("M,N,K", [(34, 1654, 752), (33, 1024, 64), (48, 2048, 1536), (64, 4096, 3072), (100, 3126, 1344)])
 def test_argmax_of_few_channels_is_fused(M, N, K):
     lib, plan = _lib.load(), GemmConfig()

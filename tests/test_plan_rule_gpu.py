@@ -15,10 +15,12 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M,N,K", [
     (1, 700, 3000), (1, 2562, 2504), (1, 4100, 4616), (2, 2050, 2560), (2, 300, 5640),   # VALU
-    (3, 515, 1032), (3, 4097, 1032), (4, 8201, 2048), (4, 2500, 3080), (8, 8300, 1000),  # VALU / wave-sliced
+    (3, 515, 1032), (3, 4097, 1032), (4, 8201, 2048), (6, 8200, 512), (8, 8203, 1536), (4, 2500, 3080), (8, 8300, 1000),  # VALU / wave-sliced
     (5, 255, 72), (12, 4096, 1416), (13, 4104, 1416), (16, 8192, 520), (32, 8200, 520), (8, 8300, 2056),
     (9, 600, 6672), (17, 1800, 4104), (24, 3300, 4104), (32, 500, 5128),                   # LDS-staged, split
     (33, 1023, 1536), (33, 1024, 3072), (64, 2047, 2048), (48, 2048, 3080), (40, 5000, 1544), (64, 9000, 1528),
+    (1, 1002, 11624), (2, 1600, 10256), (1, 3, 11272), (5, 26, 13640), (8, 36, 7888), (3, 210, 14600),  # few channels, long K
+    (7, 400, 15528), (3, 4432, 3160), (4, 16390, 3160),
     (16, 16390, 1024), (33, 16400, 1000), (33, 65536, 264), (49, 65544, 1016),              # stream
 ])
 def test_rule_plans(device, M, N, K):
@@ -28,6 +30,8 @@ def test_rule_plans(device, M, N, K):
 
 @pytest.mark.parametrize("M,I,K", [
     (1, 1025, 2824), (2, 300, 5640), (4, 2100, 1544), (6, 310, 4104), (8, 1201, 2560),     # VALU
+    (1, 300, 15752), (1, 5, 9736), (8, 24, 3504), (7, 10, 2632), (3, 1195, 14184),         # few channels, long K
+    (1, 4100, 8880), (1, 4100, 10296), (8, 850, 7176),
     (9, 4097, 520), (16, 300, 2560), (17, 2050, 4096), (32, 1300, 3600), (32, 500, 1800),  # LDS-staged
     (33, 1200, 1000), (33, 1201, 1000), (64, 4500, 1032), (40, 8300, 1032),                # stream / LDS-staged
     (36, 8200, 264), (48, 8195, 512), (64, 8200, 776), (50, 10248, 264), (64, 8199, 1016),
