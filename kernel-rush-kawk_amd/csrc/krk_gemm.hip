@@ -1353,7 +1353,11 @@ int dispatch_tile(const LaunchArgs& a, int epilogue, const TallPlan& p, hipStrea
     const krk::TileArgs t{a.x, a.ldx, a.w, a.ldw, a.y, a.ldy, a.M, a.N, a.K, p.splits, p.cb, p.nblk, a.part};
     const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
     switch (p.mt) {
-        case 4: return silu ? dispatch_tile_n<4, true>(t, p.nt, s) : dispatch_tile_n<4, false>(t, p.nt, s);
+        // 49-64 rows: only widths that take all five weight tiles (tile_width_ok).
+        case 4:
+            if (p.nt == krk::kTileMaxNT)
+                return silu ? launch_tile<4, krk::kTileMaxNT, true>(t, s) : launch_tile<4, krk::kTileMaxNT, false>(t, s);
+            return fail(KRK_ERR_UNSUPPORTED, "tile kernel of %d rows with %d weight tiles", a.M, p.nt);
         case 6: return silu ? dispatch_tile_n<6, true>(t, p.nt, s) : dispatch_tile_n<6, false>(t, p.nt, s);
         default: return silu ? dispatch_tile_n<8, true>(t, p.nt, s) : dispatch_tile_n<8, false>(t, p.nt, s);
     }

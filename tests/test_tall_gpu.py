@@ -64,7 +64,11 @@ def test_long_k_beside_too_many_channels_to_split(device, M, N, K, epi):
 ])
 def test_49_to_64_rows(device, M, N, K, epi):
     """The shapes that run on the tile kernel below 65 rows, at the ends of
-    their ranges."""
+    their ranges: 65-80 plain or 33-40 SwiGLU channels per CU under an LDS-staged
+    plan with K whole."""
+    plan, per_cu = G.plan(M, N, K, epi), -(-N // 256) / (2 if epi == SILU else 1)
+    assert plan["kernel"] == _lib.KERNEL_MFMA_LDS and plan["splits"] == 1, plan
+    assert (32 < per_cu <= 40) if epi == SILU else (64 < per_cu <= 80)
     x, w = R.randn_bf16((M, K), 9250 + M), R.randn_bf16((N, K), 9350 + N, 0.02)
     (check_gateup if epi == SILU else check_linear)(x, w, f"tile M={M} N={N} K={K}")
 
@@ -105,8 +109,8 @@ def test_special_values_stay_in_their_rows_and_columns(device, K):
     assert torch.equal(y[keep][:, :69], clean[keep][:, :69])
 
 
-def test_normed_rows_beyond_64(device):
-    M, N, K = 100, 520, 2560
+@pytest.mark.parametrize("M,N,K", [(100, 520, 2560), (64, 16400, 520), (72, 2560, 4096), (130, 70, 1032)])
+def test_normed_rows_beyond_64(device, M, N, K):
     say("normed", M, N, K)
     x, d = R.randn_bf16((M, K), 9800), R.randn_bf16((M, K), 9801)
     wn = R.randn_bf16((K,), 9802, 0.1) + 1.0
