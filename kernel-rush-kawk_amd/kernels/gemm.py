@@ -322,7 +322,6 @@ class SkinnyMatmul:
         if M < 1 or N < 1 or K < 8 or K % 8:
             raise ValueError(f"unsupported shape M={M} N={N} K={K} (need K >= 8, K % 8 == 0)")
         self.M, self.N, self.K = M, N, K
-        self._a_shape = (M, K)
         self.device = torch.device(device)
         triton_args = dict(block_n=block_n, block_k=block_k, split_k=split_k, num_warps=num_warps,
                            num_stages=num_stages)
@@ -342,7 +341,7 @@ class SkinnyMatmul:
 
     def run(self, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, norm=None) -> torch.Tensor:
         """Allocation-free form: write into ``out``."""
-        if a.shape != self._a_shape and (a.shape[0] != self.M or a.shape[1] != self.K) or w.shape[0] != self.N:
+        if a.shape != (self.M, self.K) or w.shape[0] != self.N:
             raise ValueError(f"operands {tuple(a.shape)} x {tuple(w.shape)} do not match the "
                              f"({self.M}, {self.N}, {self.K}) this object was built for")
         return gemm_into(a, w, out, self.epilogue, self.workspace, self.config, norm)

@@ -42,3 +42,19 @@ def test_other_entry_points_refuse_cpu_tensors():
         G.SkinnyMatmul(3, 8, 64, "cpu")(x, w)
     with pytest.raises(ValueError, match="w_norm"):
         G.add_rms_norm(x, _t(2, 64), _t(72), 1e-6)
+
+
+def test_projection_objects_check_their_own_sizes():
+    """The sizes of a call are the object's M, N and K, whatever else it was
+    built with: an object that lacks later attributes (pickled by an earlier
+    version), or whose M was changed, refuses what does not fit it."""
+    op = G.SkinnyMatmul.__new__(G.SkinnyMatmul)
+    op.__dict__.update(M=2, N=8, K=64, config=None, workspace=None, out_cols=8)
+    with pytest.raises(ValueError, match="must be a GPU tensor"):
+        op(_t(2, 64), _t(8, 64))
+    op.M = 3
+    with pytest.raises(ValueError, match="do not match"):
+        op(_t(2, 64), _t(8, 64))
+    for a in (_t(3, 72), _t(3, 64, 1)):
+        with pytest.raises(ValueError):
+            op(a, _t(8, 64))
