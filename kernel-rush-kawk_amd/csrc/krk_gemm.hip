@@ -494,10 +494,7 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
     // plan) unless both K and the channels are large, where the LDS-staged
     // kernel takes x in longer runs (6810 x 7120, M = 16: 21.3 against 24.4),
     // or K is long for 9-32 rows (400 x 9728, M = 32: 8.6 with 8 LDS-staged
-    // splits, over 10.8 here; 1984 x 9880, M = 15: 13.6 against 15.3; two x tiles
-    // past K = 4096 below 6 channels per CU: 512 x 4608, M = 32: 7.7 against 8.7,
-    // but 1536: 9.4 against 9.2, 3584: 13.0 against 11.3, with M = 18 12.8
-    // against 9.5).
+    // splits, over 10.8 here; 1984 x 9880, M = 15: 13.6 against 15.3).
     const int per_cu = cdiv(N, kCuCount);
     // A handful of blocks that each walk a long K, and few channels past K =
     // 11264 (3-4 rows) or 13824, go to the VALU kernel, which splits it (26 x
@@ -510,7 +507,7 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
                           (K > 3072 || (K > 1024 && K % krk::kValuBlock != 0));
     const bool sliced = Mc >= 5 && Mc <= 32 && per_cu <= kSliceMaxChannels && !(per_cu > 16 && K > 4096) && !narrow &&
                         !(Mc > 8 && K > 6656) &&
-                        !(Mc > 16 && (K > 5120 || (K > 4096 && per_cu < 6)));
+                        !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 8 || per_cu > 12))));
     const bool wide_sliced = Mc >= 5 && Mc <= 8 && per_cu > kSliceMaxChannels && K >= 2048 && K <= 8192;
     if (few_rows || sliced || wide_sliced) {
         c->kernel = KRK_KERNEL_SLICE;
