@@ -494,7 +494,12 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
     // plan) unless both K and the channels are large, where the LDS-staged
     // kernel takes x in longer runs (6810 x 7120, M = 16: 21.3 against 24.4),
     // or K is long for 9-32 rows (400 x 9728, M = 32: 8.6 with 8 LDS-staged
-    // splits, over 10.8 here; 1984 x 9880, M = 15: 13.6 against 15.3).
+    // splits, over 10.8 here; 1984 x 9880, M = 15: 13.6 against 15.3).  Two x
+    // tiles past K = 4096: from 6 channels per CU (512 x 4608, M = 32: 7.7 on the
+    // LDS-staged kernel, 8.7 here) where rows stay 64-byte aligned (K % 32 = 0:
+    // 0.94-1.3x as fast over 50 shapes); where they do not, only up to 24 rows of
+    // 12 channels (0.96-1.7x over 71 shapes; but 3208 x 5016, M = 32: 13.8 against
+    // 16.1 here).
     const int per_cu = cdiv(N, kCuCount);
     // A handful of blocks that each walk a long K, and few channels past K =
     // 11264 (3-4 rows) or 13824, go to the VALU kernel, which splits it (26 x
@@ -503,11 +508,12 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
     const bool narrow = Mc <= 4 ? (K > 7000 && N * 320 < K) || (K > 11264 && N > 128 && N <= 768)
                                 : Mc <= kValuMaxRows && ((K > 7000 && N * 192 < K) ||
                                                          (K > 13824 && N >= 256 && N <= 768));
+    const bool aligned = K % 32 == 0;
     const bool few_rows = Mc >= 3 && Mc <= 4 && N <= 16 * kCuCount && !narrow &&
                           (K > 3072 || (K > 1024 && K % krk::kValuBlock != 0));
     const bool sliced = Mc >= 5 && Mc <= 32 && per_cu <= kSliceMaxChannels && !(per_cu > 16 && K > 4096) && !narrow &&
                         !(Mc > 8 && K > 6656) &&
-                        !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 8 || per_cu > 12))));
+                        !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 6 || !(aligned || (Mc <= 24 && per_cu <= 12))))));
     const bool wide_sliced = Mc >= 5 && Mc <= 8 && per_cu > kSliceMaxChannels && K >= 2048 && K <= 8192;
     if (few_rows || sliced || wide_sliced) {
         c->kernel = KRK_KERNEL_SLICE;

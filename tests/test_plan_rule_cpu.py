@@ -104,6 +104,18 @@ def test_depth_past_one_pass(M, N, K, epi, depth):
     assert plan.kernel == _lib.KERNEL_VALU and plan.unroll == depth, plan.as_dict()
 
 
+@pytest.mark.parametrize("M,N,K,sliced", [
+    (18, 1536, 4224, True), (32, 3584, 4608, True), (24, 4096, 5120, True), (32, 2560, 5120, True),
+    (32, 512, 4608, False), (24, 4352, 4608, False), (32, 2560, 5632, False),
+    (32, 2838, 4512, True),
+    (24, 1540, 4232, True), (24, 3072, 5112, True), (25, 2560, 4408, False), (24, 3208, 5016, False),
+])
+def test_two_x_tiles_past_k_4096(M, N, K, sliced):
+    plan = GemmConfig()
+    assert _lib.load().krk_gemm_plan(M, N, K, NONE, ctypes.byref(plan)) == 0
+    assert plan.kernel == (_lib.KERNEL_SLICE if sliced else _lib.KERNEL_MFMA_LDS), plan.as_dict()
+
+
 @pytest.mark.parametrize("M,N,K,waves,rows", [
     (6, 65536, 512, 4, 2), (8, 10240, 1536, 4, 2), (8, 65536, 1024, 8, 2), (4, 65536, 512, 8, 2),
     (3, 4432, 3160, 4, 1), (3, 16390, 3160, 8, 2), (3, 8982, 3584, 8, 2),
