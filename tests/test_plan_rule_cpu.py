@@ -104,6 +104,22 @@ def test_depth_past_one_pass(M, N, K, epi, depth):
     assert plan.kernel == _lib.KERNEL_VALU and plan.unroll == depth, plan.as_dict()
 
 
+@pytest.mark.parametrize("M,N,K,stream", [
+    (72, 132988, 520, True), (45, 114926, 688, True), (83, 158058, 512, True), (64, 144730, 200, False), (64, 65522, 520, False),
+])
+def test_selecting_calls_plan_for_aligned_logits(M, N, K, stream):
+    """The workspace's rows of logits are aligned, whatever N is; a call with
+    N one short of a multiple of 8 runs the plan of that multiple."""
+    lib, plan, whole = _lib.load(), GemmConfig(), GemmConfig()
+    for k in (1, 8):
+        assert lib.krk_gemm_select_plan(M, N, K, k, ctypes.byref(plan)) == 0
+        assert (plan.kernel == _lib.KERNEL_STREAM) == stream, plan.as_dict()
+        if stream:
+            assert lib.krk_gemm_select_plan(M, -(-N // 8) * 8, K, k, ctypes.byref(whole)) == 0
+            assert plan.as_dict() == whole.as_dict()
+            assert lib.krk_gemm_select_fused(M, N, K, k, None) == lib.krk_gemm_select_fused(M, N, K, k, ctypes.byref(plan))
+
+
 @pytest.mark.parametrize("M,N,K,sliced", [
     (18, 1536, 4224, True), (32, 3584, 4608, True), (24, 4096, 5120, True), (32, 2560, 5120, True),
     (32, 512, 4608, False), (24, 4352, 4608, False), (32, 2560, 5632, False),

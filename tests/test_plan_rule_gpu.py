@@ -57,3 +57,16 @@ def test_fused_argmax_of_few_channels(device, M, N, K):
     assert_parity(logits[:M - 1], R.linear_bf16(x[:M - 1], w), "logits")
     again, _, _ = krk_select(x, w, 1, logits=False)
     assert again.tolist() == idx.tolist()
+
+
+@pytest.mark.parametrize("M,N,K,k", [(70, 65537, 264, 1), (33, 65541, 520, 8)])
+def test_selection_with_unaligned_rows(device, M, N, K, k):
+    """N not a multiple of 8: the stream kernel's logits in the aligned rows of
+    the workspace and in the caller's unaligned ones select alike."""
+    x, w = R.randn_bf16((M, K), 8700 + M), R.randn_bf16((N, K), 8800 + K, 0.02)
+    say("selection, unaligned rows", M, N, K, k)
+    idx, vals, logits = krk_select(x, w, k)
+    _check_selection(idx, vals, logits, k, f"select M={M} N={N} K={K} k={k}")
+    assert_parity(logits, R.linear_bf16(x, w), "logits")
+    again, v2, _ = krk_select(x, w, k, logits=False)
+    assert again.tolist() == idx.tolist() and v2.tolist() == vals.tolist()
