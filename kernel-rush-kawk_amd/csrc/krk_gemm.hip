@@ -499,7 +499,8 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
     // LDS-staged kernel, 8.7 here) where rows stay 64-byte aligned (K % 32 = 0:
     // 0.94-1.3x as fast over 50 shapes); where they do not, only up to 24 rows of
     // 12 channels (0.96-1.7x over 71 shapes; but 3208 x 5016, M = 32: 13.8 against
-    // 16.1 here).
+    // 16.1 here).  Nor are such rows past K = 2816 with more than 24 channels per
+    // CU at 25-32 rows (7844 x 3920, M = 32: 17.5 against 20.0 here).
     const int per_cu = cdiv(N, kCuCount);
     // A handful of blocks that each walk a long K, and few channels past K =
     // 11264 (3-4 rows) or 13824, go to the VALU kernel, which splits it (26 x
@@ -513,7 +514,8 @@ void rule_config(int Mc, int N, int K, bool silu, krk_gemm_config* c) {
                           (K > 3072 || (K > 1024 && K % krk::kValuBlock != 0));
     const bool sliced = Mc >= 5 && Mc <= 32 && per_cu <= kSliceMaxChannels && !(per_cu > 16 && K > 4096) && !narrow &&
                         !(Mc > 8 && K > 6656) &&
-                        !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 6 || !(aligned || (Mc <= 24 && per_cu <= 12))))));
+                        !(Mc > 16 && (K > 5120 || (K > 4096 && (per_cu < 6 || !(aligned || (Mc <= 24 && per_cu <= 12)))))) &&
+                        !(Mc > 24 && K > 2816 && per_cu > 24 && !aligned);
     const bool wide_sliced = Mc >= 5 && Mc <= 8 && per_cu > kSliceMaxChannels && K >= 2048 && K <= 8192;
     if (few_rows || sliced || wide_sliced) {
         c->kernel = KRK_KERNEL_SLICE;

@@ -124,9 +124,10 @@ def test_selecting_calls_plan_for_aligned_logits(M, N, K, stream):
     (18, 1536, 4224, True), (32, 3584, 4608, True), (24, 4096, 5120, True), (32, 2560, 5120, True),
     (32, 512, 4608, False), (24, 4352, 4608, False), (32, 2560, 5632, False),
     (32, 2838, 4512, True),
+    (30, 8126, 3352, False), (32, 6992, 3384, False), (30, 8126, 3360, True), (30, 8126, 2712, True), (24, 8126, 3352, True),
     (24, 1540, 4232, True), (24, 3072, 5112, True), (25, 2560, 4408, False), (24, 3208, 5016, False),
 ])
-def test_two_x_tiles_past_k_4096(M, N, K, sliced):
+def test_two_x_tiles_of_a_long_k(M, N, K, sliced):
     plan = GemmConfig()
     assert _lib.load().krk_gemm_plan(M, N, K, NONE, ctypes.byref(plan)) == 0
     assert plan.kernel == (_lib.KERNEL_SLICE if sliced else _lib.KERNEL_MFMA_LDS), plan.as_dict()

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     (1, 700, 3000), (1, 2562, 2504), (1, 4100, 4616), (2, 2050, 2560), (2, 300, 5640),   # VALU
     (3, 515, 1032), (3, 4097, 1032), (4, 8201, 2048), (6, 8200, 512), (8, 8203, 1536), (4, 2500, 3080), (8, 8300, 1000),  # VALU / wave-sliced
     (5, 255, 72), (12, 4096, 1416), (13, 4104, 1416), (16, 8192, 520), (32, 8200, 520), (8, 8300, 2056),
-    (18, 1530, 4224), (32, 4096, 5120), (24, 1540, 4616), (17, 3072, 5112),                # wave-sliced, two x tiles
+    (18, 1530, 4224), (32, 4096, 5120), (24, 1540, 4616), (17, 3072, 5112), (30, 8126, 3352),                # wave-sliced, two x tiles
     (9, 600, 6672), (17, 1800, 4104), (24, 3300, 4104), (32, 500, 5128),                   # LDS-staged, split
     (33, 1023, 1536), (33, 1024, 3072), (64, 2047, 2048), (48, 2048, 3080), (40, 5000, 1544), (64, 9000, 1528),
     (1, 1002, 11624), (2, 1600, 10256), (1, 3, 11272), (5, 26, 13640), (8, 36, 7888), (3, 210, 14600),  # few channels, long K
