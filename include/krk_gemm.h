@@ -64,12 +64,15 @@ enum {
  *   y          [M, Nout] bf16, row stride ldy >= Nout; must not overlap x, w or workspace
  *   M >= 1, N >= 1, K >= 8, K % 8 == 0.  More than 64 rows run in launches of
  *              up to 128 rows while more than 64 are left (the tile kernel, one
- *              pass over w each), then one of up to 64
+ *              pass over w each), then one of up to 64; a few shapes with a long
+ *              K run 64 rows at a time
  *   epilogue   KRK_EPILOGUE_NONE or KRK_EPILOGUE_SILU_MUL
  *   workspace  device memory of at least krk_gemm_workspace_bytes(M, N, K, epilogue)
  *              bytes (may be NULL when that is 0).  It must be zero-filled once
- *              before its first use; every call leaves it zero-filled again.
- *              Calls that share one workspace must be ordered on one stream.
+ *              before its first use; every call leaves its block counters, at
+ *              the start, zero again and sums behind them.  Calls that share
+ *              one workspace must be ordered on one stream; for another shape or
+ *              configuration it is zero-filled again first.
  *   stream     hipStream_t (NULL = the default stream)
  *
  * Results are deterministic: the same inputs and shape give bit-identical y.
@@ -306,7 +309,11 @@ int krk_add_rms_norm_bf16(const void* x, int64_t ldx, const void* d, int64_t ldd
  * outputs to one key per row and workgroup and the logits are not written
  * unless y is given; otherwise the plain projection writes the logits (to y,
  * or to the workspace) and a selection kernel reads them back.  Either way
- * the call is two kernels on one stream.
+ * a call of up to 64 rows is two kernels on one stream; more rows run 64 at a
+ * time.  Where krk_gemm_bf16 runs on the tile kernel (more than 64 rows, and
+ * some widths at 49 to 64), its fp32 sums have another order than this call's,
+ * so a logit next to a bf16 rounding boundary can differ between the two; idx
+ * and vals are those of this call's own logits.
  *
  * Replaces `logits.argmax(dim=-1)` (k = 1; engine/engine.py:196,
  * engine/model.py:365; lowest index on ties, OPTIMIZATION_GUIDE.md:213) and

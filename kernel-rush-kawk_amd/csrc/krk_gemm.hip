@@ -272,9 +272,10 @@ inline int default_kc(int MT, int NT) { return krk::mfma_lds_kc_ok(MT, NT, 512) 
 // other models' projections).  From sweeps of every candidate on 23 shapes
 // (N 400-38000, K 1024-9728, plain and SwiGLU) at 1-64 rows on an MI355X,
 // graph replay over rotating weights; times below in us.  Against the rule
-// before it, which split K until 200-600 workgroups ran, 500 random shapes
-// (N 256-24576, K 512-10240, 1-64 rows) run 1.33x as fast (geometric mean),
-// none of them more than 3% slower.
+// before it (filler_config), which split K until 200-600 workgroups ran, 1472
+// random shapes (N 64-160000, K 128-12288, 1-64 rows) run 1.19x as fast
+// (geometric mean), the worst 0.95x; of 500 of up to 8 rows, few channels and a
+// K up to 16000 the worst runs 0.92x.
 //
 // All rules cut the channels into one block per CU, or into whole rounds of
 // 256 blocks, and leave K whole: a split pays 3.4 us (2 splits) to 8 us (8)
@@ -631,8 +632,10 @@ struct TallPlan {
 // together per us, a launch costs 3 us beside that, and a split K the second
 // launch's 4 us.  The model puts qkv, gate_up and lm_head on whole K (qkv
 // M = 128: 17.0 us against 18.4 with 2 splits) and o and down on the most
-// splits their workspace holds (o: 16.2 with 4 splits, 24 unsplit).  Blocks
-// are cut to one per CU where the tiles allow it.
+// splits the scratch holds, 3 at 128 rows (o 14.6, two launches of 64 rows
+// 23.8) and 4 at 96 (13.1, 23.1).  Blocks are cut to one per CU where the tiles
+// allow it.  Over 1150 shapes the time was 0.7-1.5 of the model's, shapes of
+// few channels below it and short K above.
 TallPlan tall_plan(int rows, int N, int K, int epilogue, size_t part_bytes) {
     const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
     const int Nout = silu ? N / 2 : N;
@@ -674,7 +677,7 @@ inline size_t cut_bytes(const TallPlan& p) {
 // two splits of whole tiles do not fit (97-128 rows of 4033-4096 plain or
 // 2017-2048 SwiGLU channels) a long K goes to launches of 64, which split it:
 // 4096 x 7320, 128 rows 42.7 us against 44.2; 4080 x 11600 59.0 against 66.2; but
-// 4066 x 6112, 97 rows 36.7 against 33.2.  Over 1950 shapes of 65-128 rows no
+// 4066 x 6112, 97 rows 36.7 against 33.2.  Over 1450 shapes of 65-128 rows no
 // other loses more than 3%.
 constexpr size_t kTallPartMax = KRK_NOALLOC_SCRATCH_BYTES - KRK_NOALLOC_COUNTER_BYTES;
 constexpr int kTallWholeMaxK = 6656;

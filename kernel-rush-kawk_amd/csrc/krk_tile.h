@@ -8,20 +8,18 @@
 // leaves these row counts to cuBLAS (a tree of 4 rows for each of 32
 // sequences, engine/engine.py:501, 571-576).
 //
-// What bounds it (measured on an MI355X, N x K the Qwen3-4B projections):
-//   * a CU takes in ~120 B/ns of x from L2 and ~28 B/ns of W from HBM when
-//     it reads only one of them, but ~50 B/ns of a mix: its loads return in
-//     order, so x waits behind W.  At 128 rows a workgroup that keeps K whole
-//     reads more x than W, so the time follows the bytes each CU takes in,
-//     (rows + channels) x K of its split, and splitting K, which shrinks x's
-//     share, pays for a second launch only where channels per CU are few
-//     (o, down);
-//   * the loop without its loads takes 17 us of gate_up's 29 us at 128 rows,
-//     the loads without the MFMAs 25 us: they overlap because a wave reads
-//     its next fragments, across the stage's barrier, before it multiplies
-//     the present ones (without that: 32.9 us).
-// Against two launches of 64 rows, M = 128: qkv 25 -> 17 us, gate_up 49 ->
-// 29 us, down 36 -> 24 us, o 24 -> 16 us, lm_head 274 -> 223 us.
+// What bounds it (measured on an MI355X, N x K the Qwen3-4B projections, 128
+// rows): the stage loop without loads (LDS fragment reads, MFMAs, a barrier per
+// 128 k) takes 17.1 us of gate_up's 32.3 and 8.0 of qkv's 17.2, x loads alone
+// add 4 us to it, W loads alone 3-6, both 9-15: a CU takes in 32-49 B/ns of the
+// mix, W from HBM and x from L2.  At 128 rows a workgroup that keeps K whole
+// reads more x than W, so the time follows the bytes each CU takes in, (rows +
+// channels) x K of its split, and splitting K, which shrinks x's share, pays
+// for a second launch (4.5 us) only where channels per CU are few (o, down).  A
+// wave reads its next fragments, across the stage's barrier, before it
+// multiplies the present ones (gate_up 3-4 us faster).
+// Against two launches of 64 rows, M = 128: qkv 25.1 -> 17.6 us, gate_up 49.2 ->
+// 33.2, down 36.6 -> 24.7, o 23.8 -> 14.6, lm_head 268 -> 230.
 //
 // Work split: a workgroup owns `cb` output channels (NT tiles of 16 W rows;
 // SILU: 8 gate and the matching 8 up rows per tile, as in the stream kernel)
@@ -38,7 +36,7 @@
 // Split K: the fp32 sums go to `part` in fragment order (whole 1 KB runs) and
 // tile_reduce_kernel adds the splits in order s = 0, 1, ... in a second
 // launch.  (The in-kernel fix-up of krk_epilogue.h makes one workgroup per
-// block read every split's sums: at 8 splits it cost 7-8 us, this launch 5.)
+// block read every split's sums: at 8 splits it cost 7-8 us, this launch 4.5.)
 //
 // Rows past M and channels past the block load clamped in-range rows, whose
 // outputs are not stored; k past K is zeroed in both operands.

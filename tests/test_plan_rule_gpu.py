@@ -5,6 +5,7 @@ against the oracle."""
 from __future__ import annotations
 
 import pytest
+import torch
 
 from kernels import gemm as G
 from oracle import gemm_ref as R
@@ -55,6 +56,9 @@ def test_fused_argmax_of_few_channels(device, M, N, K):
     idx, vals, logits = krk_select(x, w, 1)
     _check_selection(idx, vals, logits, 1, f"argmax M={M} N={N} K={K}")
     assert_parity(logits[:M - 1], R.linear_bf16(x[:M - 1], w), "logits")
+    if M <= 64:  # the plain call's logits bit for bit
+        plain = check_linear(x[:M - 1], w, "plain") if M - 1 > 32 else None
+        assert plain is None or torch.equal(plain, logits[:M - 1])
     again, _, _ = krk_select(x, w, 1, logits=False)
     assert again.tolist() == idx.tolist()
 
