@@ -959,8 +959,8 @@ int complete_config(int M, int N, int K, int epilogue, const krk_gemm_config& a,
     return KRK_OK;
 }
 
-// A caller's configuration with its zero fields filled from the plan, or
-// where that is none this build runs, from filler_config.
+// A caller's configuration with its zero fields filled from the plan, or where
+// that is none this build runs, from a simpler one.
 int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in, krk_gemm_config* out) {
     krk_gemm_config plan, a;
     auto_config(M, N, K, epilogue, &plan);
@@ -973,12 +973,24 @@ int resolve_config(int M, int N, int K, int epilogue, const krk_gemm_config* in,
         if (!in->splits && !memcmp(out, &a, sizeof a)) out->splits = plan.splits;
         return rc;
     }
-    krk_gemm_config f;
-    filler_config(M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch, N, K, epilogue == KRK_EPILOGUE_SILU_MUL, &f);
-    if (complete_config(M, N, K, epilogue, f, in, out) == KRK_OK) {
-        g_err[0] = '\0';
-        return KRK_OK;
-    }
+    // Simpler plans of the kernels that take most fields.
+    const int Mc = M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch;
+    const bool silu = epilogue == KRK_EPILOGUE_SILU_MUL;
+    krk_gemm_config bases[3];
+    filler_config(Mc, N, K, silu, &bases[0]);
+    bases[1] = krk_gemm_config{};
+    lds_rule(cdiv(Mc, 16), 4, 2, 256, silu ? 32 : 64, 1, 1, &bases[1]);
+    bases[2] = krk_gemm_config{};
+    bases[2].kernel = KRK_KERNEL_SLICE;
+    bases[2].unroll = 2;
+    bases[2].splits = 1;
+    bases[2].k_chunk = 64;
+    bases[2].channels = cdiv(N, kCuCount) < kSliceMaxChannels ? cdiv(N, kCuCount) : kSliceMaxChannels;
+    for (const krk_gemm_config& f : bases)
+        if (complete_config(M, N, K, epilogue, f, in, out) == KRK_OK) {
+            g_err[0] = '\0';
+            return KRK_OK;
+        }
     return complete_config(M, N, K, epilogue, a, in, out);  // the reason against the plan's fields
 }
 

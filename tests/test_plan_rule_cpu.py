@@ -49,6 +49,10 @@ def test_plans_resolve_to_themselves(epi):
     (12, 300, 88, NONE, {"k_chunk": 256}),                             # the plan is wave-sliced
     (4, 20, 4096, NONE, {"unroll": 5}),
     (128, 80648, 14336, SILU, {"unroll": 7, "splits": 7}),
+    (5, 68, 14336, NONE, {"splits": 1, "n_tiles": 1}),                 # the plan splits K on the VALU kernel
+    (32, 2528, 4176, NONE, {"splits": 5}),
+    (64, 127376, 656, SILU, {"splits": 3}),                            # the plan is the stream kernel, of two K stages
+    (128, 24400, 408, SILU, {"kernel": _lib.KERNEL_MFMA_LDS, "channels": 24, "splits": 2}),
 ])
 def test_partial_configurations_are_completed(M, N, K, epi, cfg):
     """A configuration that names only some fields runs where some choice of
