@@ -690,15 +690,19 @@ bool tall_cut(int M, int rows, int N, int K, int epilogue, bool split, TallPlan*
     *p = tall_plan(rows, N, K, epilogue, most);
     return !split || p->splits > 1 || K <= kTallWholeMaxK;
 }
-// The most partial sums of the launches a call of M > 64 rows may have there.
+// The most partial sums of the launches that a call of M > 64 rows has there.
 size_t tall_part(int M, int N, int K, int epilogue, bool split) {
+    constexpr int kMost = krk::kTileMaxRows;
+    TallPlan p;
     size_t most = 0;
-    for (int rows : {M < krk::kTileMaxRows ? M : krk::kTileMaxRows, M % krk::kTileMaxRows,
-                     kMaxRowsPerLaunch + M % kMaxRowsPerLaunch}) {
-        TallPlan p;
-        if (rows <= kMaxRowsPerLaunch || !tall_cut(M, rows, N, K, epilogue, split, &p)) continue;
-        if (cut_bytes(p) > most) most = cut_bytes(p);
+    int last = 0;  // rows of the last launch of more than 64, if it is not the first
+    if (tall_cut(M, M < kMost ? M : kMost, N, K, epilogue, split, &p)) {
+        most = cut_bytes(p);
+        if (M > kMost) last = M % kMost;
+    } else if (M > kMost) {
+        last = kMaxRowsPerLaunch + M % kMaxRowsPerLaunch;
     }
+    if (last > kMaxRowsPerLaunch && tall_cut(M, last, N, K, epilogue, split, &p) && cut_bytes(p) > most) most = cut_bytes(p);
     return most;
 }
 
@@ -1008,13 +1012,13 @@ bool tall_call(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
 // Workspace layout: [block counters, padded to 256 B][fp32 partials: splits x
 // Mc x N, or the tile kernel's where they are more (a multiple of 64 rows that
 // does not fit the static scratch)].
-size_t workspace_for(int M, int N, int K, int epilogue, const krk_gemm_config& c) {
+size_t workspace_for(int M, int N, int K, int epilogue, const krk_gemm_config& c, bool tall) {
     if (c.splits <= 1) return 0;
     const Geometry g = geometry(M, N, epilogue, c);
     size_t part = (size_t)c.splits * (size_t)g.Mc * (size_t)N * sizeof(float);
-    if (M > kMaxRowsPerLaunch && tall_call(M, N, K, epilogue, c)) {
-        const size_t tall = tall_part(M, N, K, epilogue, true);
-        if (tall > part) part = tall;
+    if (M > kMaxRowsPerLaunch && tall) {
+        const size_t sums = tall_part(M, N, K, epilogue, true);
+        if (sums > part) part = sums;
     }
     return align_up((size_t)g.nblocks * sizeof(uint32_t), 256) + part;
 }
@@ -1594,9 +1598,10 @@ struct WorkspaceLayout {
     size_t n_off;  // offset of the normalised rows (0 if none)
     size_t total;
 };
-WorkspaceLayout workspace_layout(int M, int N, int K, int epilogue, const krk_gemm_config& c, bool normed) {
+// tall: tall_call of the configuration.
+WorkspaceLayout workspace_layout(int M, int N, int K, int epilogue, const krk_gemm_config& c, bool normed, bool tall) {
     WorkspaceLayout l;
-    l.gemm = workspace_for(M, N, K, epilogue, c);
+    l.gemm = workspace_for(M, N, K, epilogue, c, tall);
     const bool prologue = normed && !norm_fused(M, N, K, epilogue, c);
     const size_t nbytes = frag_prologue(M, c) ? krk::frag_bytes(c.m_tiles, K) : (size_t)M * K * sizeof(uint16_t);
     l.n_off = prologue ? align_up(l.gemm, 256) : 0;
@@ -1662,7 +1667,9 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
             return fail(KRK_ERR_ALIAS, "output y may not share memory with d or w_norm");
     }
 
-    const WorkspaceLayout wl = workspace_layout(M, N, K, epilogue, c, ns != nullptr);
+    const bool fused = ns && norm_fused(M, N, K, epilogue, c);
+    const bool tall = !fused && tall_call(M, N, K, epilogue, c);
+    const WorkspaceLayout wl = workspace_layout(M, N, K, epilogue, c, ns != nullptr, tall);
     if (wl.total) {
         if (!workspace) return fail(KRK_ERR_WORKSPACE, "this plan needs a %zu-byte workspace, got none", wl.total);
         if (workspace_bytes < wl.total)
@@ -1682,7 +1689,6 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     krk::NormArgs na{};
     if (ns) na = krk::NormArgs{static_cast<const uint16_t*>(ns->d), ns->ldd, static_cast<const uint16_t*>(ns->w_norm),
                                ns->eps, static_cast<uint16_t*>(ns->xout), ns->ldxo};
-    const bool fused = ns && norm_fused(M, N, K, epilogue, c);
     // Projection input: x itself, or the normalised rows a prologue kernel
     // writes into the workspace.
     const uint16_t* xin = static_cast<const uint16_t*>(x);
@@ -1710,7 +1716,6 @@ int gemm_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, i
     // More than 64 rows under the plan (a configuration equal to it included):
     // launches of up to 128 rows on the tile kernel while more than 64 are left.
     // 49 to 64 rows: one launch of it where tile_rows_ok says so.
-    const bool tall = !fused && tall_call(M, N, K, epilogue, c);
     if (tall) {  // the plan's launches of up to 64 rows
         krk_gemm_config l;
         launch_config(M, N, K, epilogue, &l);
@@ -1887,7 +1892,7 @@ SelectLayout select_layout(int M, int N, int K, int k, const SelectPlan& p) {
     const int Mc = M < kMaxRowsPerLaunch ? M : kMaxRowsPerLaunch;
     SelectLayout l;
     l.proj = (size_t)krk::kSelMaxRows * krk::kSelCtrStride * sizeof(uint32_t);
-    size_t at = align_up(l.proj + workspace_for(Mc, N, K, KRK_EPILOGUE_NONE, p.c), 256);
+    size_t at = align_up(l.proj + workspace_for(Mc, N, K, KRK_EPILOGUE_NONE, p.c, false), 256);
     l.src = at;
     if (p.fused) {
         // One key per row and projection workgroup (the stream kernel's
@@ -2105,7 +2110,7 @@ size_t krk_gemm_normed_workspace_bytes(int M, int N, int K, int epilogue, const 
     if (check_shape(M, N, K, epilogue)) return 0;
     krk_gemm_config c;
     if (resolve_normed(M, N, K, epilogue, cfg, &c)) return 0;
-    return workspace_layout(M, N, K, epilogue, c, true).total;
+    return workspace_layout(M, N, K, epilogue, c, true, tall_call(M, N, K, epilogue, c)).total;
 }
 
 int krk_gemm_normed_fused(int M, int N, int K, int epilogue, const krk_gemm_config* cfg) {
@@ -2229,14 +2234,14 @@ size_t krk_gemm_workspace_bytes(int M, int N, int K, int epilogue) {
     if (check_shape(M, N, K, epilogue)) return 0;
     krk_gemm_config c;
     auto_config(M, N, K, epilogue, &c);
-    return workspace_for(M, N, K, epilogue, c);
+    return workspace_for(M, N, K, epilogue, c, true);
 }
 
 size_t krk_gemm_config_workspace_bytes(int M, int N, int K, int epilogue, const krk_gemm_config* cfg) {
     if (check_shape(M, N, K, epilogue)) return 0;
     krk_gemm_config c;
     if (resolve_config(M, N, K, epilogue, cfg, &c)) return 0;
-    return workspace_for(M, N, K, epilogue, c);
+    return workspace_for(M, N, K, epilogue, c, tall_call(M, N, K, epilogue, c));
 }
 
 int krk_gemm_resolve(int M, int N, int K, int epilogue, const krk_gemm_config* cfg, krk_gemm_config* out) {
